@@ -8,6 +8,8 @@
 //
 // HBM-bound: one thread moves 16 codes (one 16-byte load) and writes 16 BF16
 // (two 16-byte non-temporal stores); a 256-thread block covers 256*16 channels.
+#include <algorithm>
+
 #include "q6moe_api.h"
 #include "q6moe_device.h"
 
@@ -118,13 +120,20 @@ __global__ void kv_read_scalar_kernel(KvParams p, int64_t total) {
 
 // ---------------------------------------------------------------------------
 // Quantise and write (quantize / write_quantized, attention_cache.py:15-43).
-// One thread per (row, group): max|g|, the scale, then the group's codes.
+// 2^lg lanes per (row, group): max|g| over the lanes, the scale, then each
+// lane's codes. A decode step writes 8 rows of 4 groups, so the call is bound
+// by its chain of memory round trips: with the group spread over lanes it is
+// the row's slot, its page and one load of x (one thread per group read its
+// 128 values one after another, twice: 42.4 us per call; this form 4.0 us).
+// A long quantize is bound by HBM: 16-byte loads and 8-byte stores that are
+// contiguous over the wave.
 // ---------------------------------------------------------------------------
 struct KvQuant {
   const void* x;
   int x_bf16;
   int64_t chans, group, groups;
   int scale_bf16;
+  int lg;  // log2 of the lanes per group
 };
 
 __device__ __forceinline__ float kv_x(const KvQuant& q, int64_t i) {
@@ -132,22 +141,66 @@ __device__ __forceinline__ float kv_x(const KvQuant& q, int64_t i) {
                   : reinterpret_cast<const float*>(q.x)[i];
 }
 
-// Quantise group g of row r into codes (chans-strided destination) and
-// return the stored scale value (FP32 holding the BF16 or FP32 scale).
-__device__ __forceinline__ float kv_quant_group(const KvQuant& q, int64_t r, int64_t g, int8_t* dst) {
-  const int64_t base = r * q.chans + g * q.group;
-  float m = 0.f;
-  for (int64_t c = 0; c < q.group; ++c) m = fmaxf(m, fabsf(kv_x(q, base + c)));
-  float scale = m / 127.f;
-  if (q.scale_bf16) scale = bf16_round(scale);
-  const float divisor = scale == 0.f ? 1.f : scale;
-  for (int64_t c = 0; c < q.group; ++c) {
-    float v = __builtin_rintf(kv_x(q, base + c) / divisor);
-    v = fminf(fmaxf(v, -127.f), 127.f);
-    dst[c] = (int8_t)(int)v;
-  }
-  return scale;
+// The stored scale of a group of maximum ``m`` (FP32 holding the BF16 or FP32
+// value), and the code of a value.
+__device__ __forceinline__ float kv_group_scale(const KvQuant& q, float m) {
+  for (int off = 1; off < 1 << q.lg; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+  const float scale = m / 127.f;
+  return q.scale_bf16 ? bf16_round(scale) : scale;
 }
+__device__ __forceinline__ int kv_code(float x, float divisor) {
+  const float v = fminf(fmaxf(__builtin_rintf(x / divisor), -127.f), 127.f);
+  return (int)v;
+}
+
+// The lane's values of one group. kVec: 8 consecutive values per lane, the
+// group exactly covered (vector loads and stores); otherwise the lane takes
+// positions lane, lane + 2^lg, ... one at a time.
+template <bool kVec>
+struct KvGroup;
+
+template <>
+struct KvGroup<true> {
+  float v[8];
+  __device__ __forceinline__ float load(const KvQuant& q, int64_t base, int l) {
+    const int64_t at = base + 8 * l;
+    if (q.x_bf16) {
+      const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(q.x) + at);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = bf16_to_float((uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+    } else {
+      const f32x4* p = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(q.x) + at);
+      const f32x4 a = p[0], b = p[1];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = a[i];
+        v[4 + i] = b[i];
+      }
+    }
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));
+    return m;
+  }
+  __device__ __forceinline__ void store(const KvQuant&, int64_t, int l, float divisor, int8_t* dst) const {
+    u32x2 w = {0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i >> 2] |= ((uint32_t)kv_code(v[i], divisor) & 0xffu) << (8 * (i & 3));
+    *reinterpret_cast<u32x2*>(dst + 8 * l) = w;
+  }
+};
+
+template <>
+struct KvGroup<false> {
+  __device__ __forceinline__ float load(const KvQuant& q, int64_t base, int l) {
+    float m = 0.f;
+    for (int64_t c = l; c < q.group; c += 1 << q.lg) m = fmaxf(m, fabsf(kv_x(q, base + c)));
+    return m;
+  }
+  __device__ __forceinline__ void store(const KvQuant& q, int64_t base, int l, float divisor, int8_t* dst) const {
+    for (int64_t c = l; c < q.group; c += 1 << q.lg) dst[c] = (int8_t)kv_code(kv_x(q, base + c), divisor);
+  }
+};
 
 __device__ __forceinline__ void kv_store_scale(void* scales, int bf16, int64_t idx, float v) {
   if (bf16)
@@ -156,12 +209,17 @@ __device__ __forceinline__ void kv_store_scale(void* scales, int bf16, int64_t i
     reinterpret_cast<float*>(scales)[idx] = v;
 }
 
+template <bool kVec>
 __global__ void __launch_bounds__(256) kv_quantize_kernel(KvQuant q, int64_t rows, int8_t* codes, void* scales) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * q.groups) return;
-  const int64_t r = i / q.groups, g = i % q.groups;
-  const float s = kv_quant_group(q, r, g, codes + r * q.chans + g * q.group);
-  kv_store_scale(scales, q.scale_bf16, i, s);
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = (int)(t & ((1 << q.lg) - 1));
+  for (int64_t i = t >> q.lg; i < rows * q.groups; i += ((int64_t)gridDim.x * blockDim.x) >> q.lg) {  // (row, group)
+    const int64_t base = i * q.group;  // rows hold whole groups
+    KvGroup<kVec> g;
+    const float scale = kv_group_scale(q, g.load(q, base, l));
+    g.store(q, base, l, scale == 0.f ? 1.f : scale, codes + base);
+    if (l == 0) kv_store_scale(scales, q.scale_bf16, i, scale);
+  }
 }
 
 struct KvWrite {
@@ -174,23 +232,48 @@ struct KvWrite {
   const uint8_t* active;
 };
 
+template <bool kVec>
 __global__ void __launch_bounds__(256) kv_write_kernel(KvQuant q, KvWrite w, int64_t batch) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= batch * q.groups) return;
-  const int64_t b = i / q.groups, g = i % q.groups;
-  if (w.active && !w.active[b]) return;
-  int64_t t = w.indices[b];
-  if (t < 0) t += w.cap;
-  if (t < 0 || t >= w.cap) return;  // out-of-bounds scatter updates are dropped
-  int64_t row = b * w.cap + t;
-  if (w.table) {
-    const int64_t pg = w.table[b * w.pps + t / w.page];
-    if (pg < 0 || pg >= w.pool_pages) return;
-    row = pg * w.page + t % w.page;
+  const int64_t th = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int l = (int)(th & ((1 << q.lg) - 1));
+  for (int64_t i = th >> q.lg; i < batch * q.groups; i += ((int64_t)gridDim.x * blockDim.x) >> q.lg) {  // (row, group)
+    const int64_t b = i / q.groups, g = i % q.groups;
+    int64_t t = w.indices[b];
+    const bool on = !w.active || w.active[b];
+    KvGroup<kVec> x;
+    const float m = x.load(q, i * q.group, l);
+    if (t < 0) t += w.cap;
+    if (!on || t < 0 || t >= w.cap) continue;  // out-of-bounds scatter updates are dropped
+    int64_t row = b * w.cap + t;
+    if (w.table) {
+      const int64_t pg = w.table[b * w.pps + t / w.page];
+      if (pg < 0 || pg >= w.pool_pages) continue;
+      row = pg * w.page + t % w.page;
+    }
+    const float scale = kv_group_scale(q, m);
+    x.store(q, i * q.group, l, scale == 0.f ? 1.f : scale, w.codes + row * q.chans + g * q.group);
+    if (l == 0) {
+      const int64_t idx = w.scale_plane ? (b * q.groups + g) * w.cap + t : row * q.groups + g;
+      kv_store_scale(w.scales, q.scale_bf16, idx, scale);
+    }
   }
-  const float s = kv_quant_group(q, b, g, w.codes + row * q.chans + g * q.group);
-  const int64_t idx = w.scale_plane ? (b * q.groups + g) * w.cap + t : row * q.groups + g;
-  kv_store_scale(w.scales, q.scale_bf16, idx, s);
+}
+
+// The lanes per group (log2) of a call and whether they take 8 consecutive
+// values each: groups of 8, 16, .., 512 values with x aligned for 16-byte
+// loads and codes for 8-byte stores. Other groups spread over the largest
+// power of two of lanes, at most 64, that each still have a value.
+constexpr int64_t kQuantGrid = 1 << 20;  // workgroups; more groups take more than one turn
+
+static bool kv_quant_lanes(KvQuant& q, const int8_t* codes) {
+  for (q.lg = 0; q.lg <= 6; ++q.lg)
+    if (q.group == (int64_t)8 << q.lg) {
+      if (aligned(q.x, 16) && aligned(codes, 8)) return true;
+      break;
+    }
+  q.lg = 0;
+  while (q.lg < 6 && q.group >= (int64_t)2 << q.lg) ++q.lg;
+  return false;
 }
 
 // gather_scale_plane (kaggle/qwen38_tpu/attention_cache.py:46-68): plane
@@ -239,10 +322,13 @@ extern "C" int q6moe_kv_quantize(const void* x, int x_dtype, int64_t rows, int64
                 "kv_quantize: rows, chans must be positive and group must divide chans");
   Q6MOE_REQUIRE(x_dtype == Q6MOE_BF16 || x_dtype == Q6MOE_F32, "kv_quantize: x dtype");
   Q6MOE_REQUIRE(scale_dtype == Q6MOE_BF16 || scale_dtype == Q6MOE_F32, "kv_quantize: scale dtype");
-  KvQuant q{x, x_dtype == Q6MOE_BF16, chans, group, chans / group, scale_dtype == Q6MOE_BF16};
-  const int64_t n = rows * q.groups;
-  hipLaunchKernelGGL(kv_quantize_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, q,
-                     rows, codes, scales);
+  KvQuant q{x, x_dtype == Q6MOE_BF16, chans, group, chans / group, scale_dtype == Q6MOE_BF16, 0};
+  const bool vec = kv_quant_lanes(q, codes);
+  const dim3 grid((unsigned)std::min(cdiv((rows * q.groups) << q.lg, 256), kQuantGrid));
+  if (vec)
+    hipLaunchKernelGGL(kv_quantize_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, q, rows, codes, scales);
+  else
+    hipLaunchKernelGGL(kv_quantize_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, q, rows, codes, scales);
   return check_launch("kv_quantize");
 }
 
@@ -275,10 +361,13 @@ extern "C" int q6moe_kv_write(const q6moe_kv_write_args* a, void* stream) {
     Q6MOE_REQUIRE(a->capacity >= 1, "kv_write: capacity must be positive");
     w.cap = a->capacity;
   }
-  KvQuant q{a->x, a->x_dtype == Q6MOE_BF16, chans, a->group, chans / a->group, a->scale_dtype == Q6MOE_BF16};
-  const int64_t n = a->batch * q.groups;
-  hipLaunchKernelGGL(kv_write_kernel, dim3((unsigned)cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, q, w,
-                     a->batch);
+  KvQuant q{a->x, a->x_dtype == Q6MOE_BF16, chans, a->group, chans / a->group, a->scale_dtype == Q6MOE_BF16, 0};
+  const bool vec = kv_quant_lanes(q, w.codes);
+  const dim3 grid((unsigned)std::min(cdiv((a->batch * q.groups) << q.lg, 256), kQuantGrid));
+  if (vec)
+    hipLaunchKernelGGL(kv_write_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, q, w, a->batch);
+  else
+    hipLaunchKernelGGL(kv_write_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, q, w, a->batch);
   return check_launch("kv_write");
 }
 

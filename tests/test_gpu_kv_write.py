@@ -134,3 +134,28 @@ def test_inactive_and_out_of_range_rows_leave_the_cache_unchanged(device):
     assert np.all(np.delete(k[2], 2, axis=0) == 9)
     np.testing.assert_array_equal(cache["k_scale"].float().cpu().numpy()[4:, 2], want_scale[2])
     assert np.all(cache["k_scale"].float().cpu().numpy()[:4] == 2.0)
+
+
+@pytest.mark.parametrize("group", [1, 3, 8, 12, 64, 100, 512, 1024])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_quantize_group_widths_and_alignment(device, group, dtype):
+    # one to 64 lanes per group with 8 values each (8, 64, 512), strided lanes
+    # for the other widths and for rows at an odd address; NaN and infinity
+    # take the codes of the same formula in NumPy
+    rng = np.random.default_rng(group)
+    x = bf16_round(rng.normal(size=(7, 2 * group)).astype(np.float32) * rng.uniform(0.01, 4, (7, 1)))
+    x[2] = 0
+    want_codes, want_scale = oracle_kv.quantize(x, group, "f32")
+    buf = torch.zeros(x.size + 1, dtype=dtype, device=device)
+    for shift in (0, 1):
+        view = buf[shift: shift + x.size].view(7, 2 * group)
+        view.copy_(torch.from_numpy(x).to(device))
+        codes, scale = quantize(view, group, scale_dtype=torch.float32)
+        np.testing.assert_array_equal(codes.cpu().numpy(), want_codes)
+        np.testing.assert_array_equal(scale.cpu().numpy(), want_scale)
+    special = torch.from_numpy(x).to(device).to(dtype)
+    special[0, group - 1], special[1, 0] = float("nan"), float("inf")
+    codes, scale = (t.cpu().numpy() for t in quantize(special, group, scale_dtype=torch.float32))
+    assert codes[0, group - 1] == -127 and codes[1, 0] == -127 and np.isinf(scale[1, 0])
+    np.testing.assert_array_equal(codes[1, 1:group], 0)  # finite over an infinite scale
+    np.testing.assert_array_equal(codes[2:], want_codes[2:])
