@@ -201,10 +201,9 @@ int launch_dec_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStr
 bool pf_unpack_supported(int fmt);
 int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStream_t s);
 
-// Prefill grouped GEMM, tiled on the matrix cores: gate/up (Q6_K, Q8_0 or
-// Q4_K; hidden a multiple of 128, intermediate of 64) and down (Q6_K, Q8_0,
-// Q5_1 or Q4_K; intermediate a multiple of 128, hidden of 128), each launched
-// on its own.
+// Prefill grouped GEMM, tiled on the matrix cores: gate/up (every format but
+// Q5_1; hidden a multiple of 128, intermediate of 64) and down (every format;
+// intermediate a multiple of 128, hidden of 128), each launched on its own.
 bool pf_gate_up_supported(int fmt, int64_t H, int64_t I);
 bool pf_down_supported(int fmt, int64_t H, int64_t I);
 int64_t pf_tile_routes();

@@ -1,6 +1,6 @@
 // Prefill-shaped routed experts: tiled grouped GEMM on BF16 MFMA over
-// unit-major expert tables (gate/up Q6_K, Q8_0 or Q4_K; down Q6_K, Q8_0, Q5_1
-// or Q4_K).
+// unit-major expert tables (gate/up Q6_K, Q5_K, Q4_K or Q8_0; down any of them
+// or Q5_1).
 //
 // The routing kernel (moe.hip) groups the routes by expert (ascending id,
 // tokens ascending) and splits each expert's routes into tiles of 128. One
@@ -89,15 +89,19 @@ __device__ __forceinline__ void wait_vm() {
 // its first half's code words for the second instead of the zero padding);
 // ``half(h)`` gives the 4 A fragments of K half h; ``gran(f, jA)`` is the
 // 8-column granule, within the half, of fragment f for k-group jA (the token
-// operand it pairs with); ``pin`` makes the registers opaque to the compiler.
+// operand it pairs with); ``pin`` makes the registers opaque to the
+// compiler; ``fold`` runs once on arrived registers, before the first ``half``.
 template <int FMT>
 struct Block;
+struct NoFold {
+  __device__ __forceinline__ void fold(int) {}
+};
 
 // Q6_K (bit-planar unit): the lane's four code words of each of the three code
 // chunks, its sub-scale word and the row's FP16 scale. Fragment 2g + e of the
 // unit covers positions 64g + 16jA + 8e + [0, 8) (q6_xfrag_offset).
 template <>
-struct Block<FMT_Q6> {
+struct Block<FMT_Q6> : NoFold {
   static constexpr int kLoads = 5;
   u32x4 c0, c1, c2;
   uint32_t sc, d;
@@ -123,7 +127,7 @@ struct Block<FMT_Q6> {
 // positions) and the FP16 scales of its blocks 2g + jA/2; w = d * q exact,
 // RNE to BF16 (gguf_quant.py:111-114).
 template <>
-struct Block<FMT_Q8> {
+struct Block<FMT_Q8> : NoFold {
   static constexpr int kLoads = 5;
   u32x4 c[4];
   u32x2 dw;
@@ -151,7 +155,7 @@ struct Block<FMT_Q8> {
 // high-bit words and FP16 d, m; w = fma(q, d, m), one rounding, RNE to BF16
 // (kaggle/qwen38_tpu/quant.py:34-53).
 template <>
-struct Block<FMT_Q51> {
+struct Block<FMT_Q51> : NoFold {
   static constexpr int kLoads = 6;
   u32x4 q[4];
   u32x4 aux[2];  // blocks 2g + jA/2 of g = 0, 1 and of g = 2, 3: (high word, d | m << 16)
@@ -188,6 +192,25 @@ struct Block<FMT_Q51> {
   static __device__ __forceinline__ int gran(int f, int jA) { return Block<FMT_Q6>::gran(f, jA); }
 };
 
+// Scale and min of sub-block 4h + jA of a Q4_K / Q5_K header chunk (h a
+// compile-time constant after unrolling): ds = d * sc, dm = -(dmin * m)
+// (gguf_quant.py:118-135).
+__device__ __forceinline__ void k_half_scale_min(const u32x4& hdr, int h, int jA, float& ds, float& dm) {
+  const float d = half_bits_to_float(hdr[0] & 0xffff);
+  const float dmin = half_bits_to_float(hdr[0] >> 16);
+  uint32_t scb, mnb;
+  if (h == 0) {
+    scb = (hdr[1] >> (8 * jA)) & 63;
+    mnb = (hdr[2] >> (8 * jA)) & 63;
+  } else {
+    const uint32_t xb = hdr[3] >> (8 * jA);
+    scb = (xb & 15) | ((hdr[1] >> (8 * jA + 2)) & 48);
+    mnb = ((xb >> 4) & 15) | ((hdr[2] >> (8 * jA + 2)) & 48);
+  }
+  ds = d * (float)scb;
+  dm = -(dmin * (float)mnb);
+}
+
 // Q4_K, with a lane map of its own (the unit's bytes are those of the other
 // kernels): in K half h the lane decodes sub-block 4h + jA, positions
 // 128h + 32jA + [0, 32), i.e. the low (jA even) or high (jA odd) nibbles of
@@ -196,7 +219,7 @@ struct Block<FMT_Q51> {
 // codes enter v_fma_mix_f32 as FP16 subnormals (sub_frag): w = fma(q, d*sc,
 // -dmin*m), one rounding, RNE to BF16 (gguf_quant.py:115-157).
 template <>
-struct Block<FMT_Q4K> {
+struct Block<FMT_Q4K> : NoFold {
   static constexpr int kLoads = 5;
   u32x4 hdr;
   u32x4 qs[2][2];  // [half][chunk]
@@ -215,25 +238,80 @@ struct Block<FMT_Q4K> {
   }
   __device__ __forceinline__ void half(int h, int lane, u32x4 a[4]) const {
     const int jA = lane >> 4, odd = jA & 1;
-    const float d = half_bits_to_float(hdr[0] & 0xffff);
-    const float dmin = half_bits_to_float(hdr[0] >> 16);
-    // sub-block 4h + jA: its 6-bit scale and min (gguf_quant.py:118-135)
-    uint32_t scb, mnb;
-    if (h == 0) {
-      scb = (hdr[1] >> (8 * jA)) & 63;
-      mnb = (hdr[2] >> (8 * jA)) & 63;
-    } else {
-      const uint32_t xb = hdr[3] >> (8 * jA);
-      scb = (xb & 15) | ((hdr[1] >> (8 * jA + 2)) & 48);
-      mnb = ((xb >> 4) & 15) | ((hdr[2] >> (8 * jA + 2)) & 48);
-    }
-    const float ds = d * (float)scb, dm = -(dmin * (float)mnb);
+    float ds, dm;
+    k_half_scale_min(hdr, h, jA, ds, dm);
     const uint32_t m = odd ? 0x00F000F0u : 0x000F000Fu;
     const float s = ds * (odd ? 1048576.f : 16777216.f);
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const uint32_t w0 = qs[h][f >> 1][2 * (f & 1)], w1 = qs[h][f >> 1][2 * (f & 1) + 1];
       a[f] = sub_frag(w0 & m, (w0 >> 8) & m, w1 & m, (w1 >> 8) & m, s, dm);
+    }
+  }
+  static __device__ __forceinline__ int gran(int f, int jA) { return 4 * jA + f; }
+};
+
+// Q5_K, with Q4_K's lane map (in K half h the lane decodes sub-block s = 4h + jA,
+// fragment f its positions 8f + [0, 8)): nibbles in chunks 3 + 2c and 4 + 2c of
+// the unit (c = 2h + jA/2), bit s of the 32 high-bit bytes (chunks 1, 2) as bit
+// 4. ``pin`` keeps the lane's two bits per high-bit byte in two words (28
+// registers per unit while loading, 22 from then on): bit i of the low (high)
+// nibble of byte b of word p is the fifth bit of position 16p + 4i + b of K
+// half 0 (1). Nibble and fifth bit meet as FP16 subnormals (sub_frag): the
+// nibbles of bytes 0 and 2 of a code word at bits 0-3 (4-7 for an odd
+// sub-block) of its halves, the fifth bits rotated to bit 4 (8); bytes 1 and 3
+// the same after a shift by 8. w = fma(q, d*sc, -dmin*m), one rounding, RNE to
+// BF16 (gguf_quant.py:115-157).
+template <>
+struct Block<FMT_Q5K> {
+  static constexpr int kLoads = 7;
+  u32x4 hdr, qh[2];
+  u32x4 qs[2][2];  // [half][chunk]
+  __device__ __forceinline__ void load(const uint8_t* v, int lane, bool = false) {
+    const int j = lane & 15, jA = lane >> 4;
+    hdr = *reinterpret_cast<const u32x4*>(v + 16 * j);
+    qh[0] = *reinterpret_cast<const u32x4*>(v + 16 * (16 + j));
+    qh[1] = *reinterpret_cast<const u32x4*>(v + 16 * (32 + j));
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 2 * h + (jA >> 1);
+      qs[h][0] = *reinterpret_cast<const u32x4*>(v + 16 * (16 * (3 + 2 * c) + j));
+      qs[h][1] = *reinterpret_cast<const u32x4*>(v + 16 * (16 * (4 + 2 * c) + j));
+    }
+  }
+  __device__ __forceinline__ void pin() {
+    asm volatile("" : "+v"(hdr), "+v"(qh[0]), "+v"(qh[1]), "+v"(qs[0][0]), "+v"(qs[0][1]), "+v"(qs[1][0]),
+                      "+v"(qs[1][1]));
+  }
+  // the high bits of the block, once per K block, right after its first pin
+  __device__ __forceinline__ void fold(int lane) {
+    const int jA = lane >> 4;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      uint32_t v = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v |= ((qh[p][i] >> jA) & 0x11111111u) << i;
+      qh[0][p] = (jA & 1) ? __builtin_amdgcn_alignbit(v, v, 28) : v;  // odd: the target bit is 4 higher
+    }
+    asm volatile("" : "+v"(qh[0][0]), "+v"(qh[0][1]));
+  }
+  __device__ __forceinline__ void half(int h, int lane, u32x4 a[4]) const {
+    const int jA = lane >> 4, odd = jA & 1;
+    float ds, dm;
+    k_half_scale_min(hdr, h, jA, ds, dm);
+    const uint32_t m = odd ? 0x00F000F0u : 0x000F000Fu, hm = odd ? 0x01000100u : 0x00100010u;
+    const float sc = ds * (odd ? 1048576.f : 16777216.f);
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      uint32_t e[2], o[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t w = qs[h][f >> 1][2 * (f & 1) + i], b = qh[0][f >> 1];
+        const int at = 2 * (f & 1) + i + 4 * h;  // bit of the byte
+        e[i] = (w & m) | (__builtin_amdgcn_alignbit(b, b, (at - 4) & 31) & hm);
+        o[i] = ((w >> 8) & m) | (__builtin_amdgcn_alignbit(b, b, (at + 4) & 31) & hm);
+      }
+      a[f] = sub_frag(e[0], o[0], e[1], o[1], sc, dm);
     }
   }
   static __device__ __forceinline__ int gran(int f, int jA) { return 4 * jA + f; }
@@ -377,7 +455,10 @@ __device__ __forceinline__ void pf_stream(uint8_t* smem, const Proj* projs, cons
     // here so that the compiler does not also wait, after the next step's
     // loads are issued, for everything in flight before decoding them.
 #pragma unroll
-    for (int u = 0; u < kUnits; ++u) wr[set][u].pin();
+    for (int u = 0; u < kUnits; ++u) {
+      wr[set][u].pin();
+      if constexpr (slot == 0) wr[set][u].fold(lane);
+    }
     const bool more = s + 1 < S;
     const uint8_t* xs = smem + slot * kHalfBytes;
     u32x4 a[kUnits][4];
@@ -542,11 +623,11 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
 // The tiled kernels take K in halves of 128 and whole workgroup row blocks:
 // gate/up 64 intermediate rows, down 128 hidden rows.
 bool pf_gate_up_supported(int fmt, int64_t H, int64_t I) {
-  return (fmt == FMT_Q6 || fmt == FMT_Q8 || fmt == FMT_Q4K) && H % 128 == 0 && I % (16 * pf::kWaves) == 0;
+  return fmt != FMT_Q51 && H % 128 == 0 && I % (16 * pf::kWaves) == 0;
 }
 bool pf_down_supported(int fmt, int64_t H, int64_t I) {
-  return (fmt == FMT_Q6 || fmt == FMT_Q8 || fmt == FMT_Q51 || fmt == FMT_Q4K) && I % 128 == 0 &&
-         H % (32 * pf::kWaves) == 0;
+  (void)fmt;
+  return I % 128 == 0 && H % (32 * pf::kWaves) == 0;
 }
 
 int64_t pf_tile_routes() { return pf::kM; }
@@ -557,6 +638,7 @@ static void dispatch_pf_format(int fmt, F&& f) {
     case FMT_Q8: f(std::integral_constant<int, FMT_Q8>{}); break;
     case FMT_Q51: f(std::integral_constant<int, FMT_Q51>{}); break;
     case FMT_Q4K: f(std::integral_constant<int, FMT_Q4K>{}); break;
+    case FMT_Q5K: f(std::integral_constant<int, FMT_Q5K>{}); break;
     default: f(std::integral_constant<int, FMT_Q6>{}); break;
   }
 }
@@ -610,6 +692,7 @@ __global__ void __launch_bounds__(64) moe_pf_unpack_kernel(Proj p, uint16_t* __r
   const int e = blockIdx.y, rg = blockIdx.x / p.kb, kb = blockIdx.x - rg * p.kb;
   pf::Block<FMT> w;
   w.load(p.data + (int64_t)e * p.dstride + ((int64_t)rg * p.kb + kb) * UnitBytes<FMT>::value, lane);
+  w.fold(lane);
   u32x4 a[8];
   w.half(0, lane, a);
   w.half(1, lane, a + 4);

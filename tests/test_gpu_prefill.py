@@ -122,3 +122,57 @@ def test_prefill_routing_wide_top_k(device):
     got, _ = _run(L, device, mode=2, ids=ids, weights=w)
     assert np.all(got[100:110] == 0)
     assert_moe_close(got, _oracle(L, ids=ids, weights=w))
+
+
+def _q8_table(weights):
+    """Q8_0 bytes [rows, blocks, 34] of exactly representable weights: scale 0.5, codes 2 * weights."""
+    rows, width = weights.shape
+    raw = np.zeros((rows, width // 32, 34), np.uint8)
+    raw[..., :2] = np.array([0.5], np.float16).view(np.uint8)
+    raw[..., 2:] = (2 * weights).astype(np.int8).view(np.uint8).reshape(rows, width // 32, 32)
+    return raw
+
+
+def test_tiled_q5_k_weights_are_exact(device):
+    # One-hot tokens: every product sum has a single term, so no summation order
+    # matters and the outputs show each decoded weight. Gate/up: a 1:1 down
+    # projection passes the activations through, and the tiled kernel must agree
+    # bit for bit with the decode-step one, whose decoder is checked on its own.
+    # Down: one activation of 64 per token, y = RNE(64 * weight).
+    from oracle.gguf import dequantize_rows
+    from oracle.packed_q6 import bf16_round
+    from q6moe.experts import expert_parallel
+
+    rng = np.random.default_rng(55)
+
+    def q5(rows, width):
+        raw = rng.integers(0, 256, (rows, width // 256, 176), dtype=np.uint8)
+        raw[..., :4] = rng.uniform(0.01, 0.05, (rows, width // 256, 2)).astype(np.float16).view(np.uint8)
+        return raw
+
+    H = I = 512
+    eye = _q8_table(np.eye(H, dtype=np.float32))
+    x = torch.eye(H, device=device, dtype=torch.bfloat16)
+    ids = torch.zeros(H, 1, dtype=torch.int32, device=device)
+    ones = torch.ones(H, 1, device=device, dtype=torch.bfloat16)
+    fn = expert_parallel(None, gate_type="Q5_K", up_type="Q5_K", down_type="Q8_0", hidden=H, intermediate=I)
+    tabs = fn.prepare(*(t.reshape(1, -1) for t in (q5(I, H), q5(I, H), eye)), device)
+    for part in (slice(0, 256), slice(256, 512)):
+        got = fn.with_mode(2)(*tabs, x[part], ids[part], ones[part])
+        assert torch.equal(got, fn.with_mode(1)(*tabs, x[part], ids[part], ones[part])) and got.any()
+
+    raw = q5(H, I)
+    fn = expert_parallel(None, gate_type="Q8_0", up_type="Q8_0", down_type="Q5_K", hidden=H, intermediate=I)
+    gate = _q8_table(np.eye(H, dtype=np.float32) * 32)  # g = 32, silu(g) = 32 exactly; u = 2
+    tabs = fn.prepare(*(t.reshape(1, -1) for t in (gate, _q8_table(np.eye(H, dtype=np.float32) * 2), raw)), device)
+    got = fn.with_mode(2)(*tabs, x, ids, ones).float().cpu().numpy()
+    want = bf16_round(64 * bf16_round(dequantize_rows(raw, "Q5_K", I).reshape(H, I)).T)
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("down,hidden,inter", [("Q5_K", 512, 256), ("Q8_0", 384, 640), ("Q5_1", 256, 384)])
+def test_tiled_q5_k_layers(device, down, hidden, inter):
+    L = moe_layer(seed=hidden + inter, experts=6, top_k=2, hidden=hidden, intermediate=inter, tokens=300,
+                  qtype="Q5_K", down_qtype=down, bias_sigma=1.0, pack=False)
+    got, _ = _run(L, device, mode=2)
+    assert_moe_close(got, _oracle(L))
