@@ -946,15 +946,6 @@ static void launch_down(const Proj& d, const TokenSrc& src, int grid_x, int max_
                        d, src, act, I, y, H, kw2);
 }
 
-template <int FG, int FD, typename Mark>
-static void launch_phases(const Proj& g, const Proj& u, const Proj& d, const TokenSrc& src, int grid_x,
-                          int max_tokens, const uint16_t* x, int H, int I, uint16_t* act, uint16_t* y,
-                          hipStream_t s, Mark mark) {
-  launch_gate_up<FG>(g, u, src, grid_x, max_tokens, x, H, I, act, s);
-  mark(2);
-  launch_down<FD>(d, src, grid_x, max_tokens, act, H, I, y, s);
-}
-
 // ---------------------------------------------------------------------------
 // W8A8 policy for Q8_0 tables: kaggle/qwen38_tpu/compute.py:20-34 (q8_matmul).
 // The activations are quantised per row and 32-value group -- scale
@@ -1499,23 +1490,45 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     if (a->events && a->events[i]) (void)hipEventRecord((hipEvent_t)a->events[i], s);
   };
   const int fmt = fmt_of(a->gate.qtype), fmt_dn = fmt_of(a->down.qtype);
-  // Generic (non-tiled) expert phases for the call's formats.
-  auto phases = [&](const Proj& pg, const Proj& pu, const Proj& pd, const TokenSrc& src, int grid_x, int max_tok,
-                    int inter, uint16_t* act_out, uint16_t* y_out, auto mk) {
-    dispatch_formats(fmt, fmt_dn, [&](auto fg, auto fd) {
-      launch_phases<decltype(fg)::value, decltype(fd)::value>(pg, pu, pd, src, grid_x, max_tok, a->x, (int)H, inter,
-                                                              act_out, y_out, s, mk);
-    });
+  // The shared expert outside the decode launches. Its gate/up and down run
+  // tiled where the shape allows (full tiles of 128 tokens against blocks of
+  // its rows), in the routed experts' launches where those are tiled too: its
+  // few column blocks then fill the chip together with the routed items. The
+  // generic kernels, which take any shape, decode its weights again for every
+  // 64 tokens. 64-expert top-6 Q4_K layer (H 4096, I 1024, shared 4096): at
+  // 1024 tokens 868 us of generic kernels against 144 us more in the tiled
+  // launches (the step 1150 -> 379 us); at 100 tokens 107 us against 23 us.
+  const bool sh32 = B * H * 2 < (1ll << 31) && B * Is * 2 < (1ll << 31);
+  const bool sh_tiled_gu = Is && sh32 && pf_gate_up_supported(fmt, H, Is);
+  const bool sh_tiled_dn = Is && sh32 && pf_down_supported(fmt_dn, H, Is);
+  const Proj sg = make_proj(a->shared_gate, (int)Is, (int)H), su = make_proj(a->shared_up, (int)Is, (int)H),
+             sd = make_proj(a->shared_down, (int)H, (int)Is);
+  const TokenSrc dense{1, (int)B, nullptr, nullptr, nullptr, nullptr};
+  const auto shared_gate_up = [&] {  // in a launch of its own
+    if (sh_tiled_gu)
+      launch_moe_prefill_gate_up(fmt, sg, su, ws, 0, a->x, (int)B, (int)H, (int)Is,
+                                 pf_dense_gate_up(sg, su, a->x, (int)B, ws.sh_act), s, nullptr, nullptr);
+    else
+      dispatch_format(fmt, [&](auto fg) {
+        launch_gate_up<decltype(fg)::value>(sg, su, dense, 1, (int)B, a->x, (int)H, (int)Is, ws.sh_act, s);
+      });
+  };
+  const auto shared_down = [&] {
+    if (sh_tiled_dn)
+      launch_moe_prefill_down(fmt_dn, sd, ws, 0, (int)B, (int)H, (int)Is,
+                              pf_dense_down(sd, ws.sh_act, (int)B, ws.sh_y), s);
+    else
+      dispatch_format(fmt_dn, [&](auto fd) {
+        launch_down<decltype(fd)::value>(sd, dense, 1, (int)B, ws.sh_act, (int)H, (int)Is, ws.sh_y, s);
+      });
   };
   if (decode) {
     mark(0);
     // up to kDecSharedTokens tokens the shared expert runs inside the decode launches
     const bool fused_shared = Is && B <= kDecSharedTokens;
     if (Is && !fused_shared) {
-      TokenSrc dense{1, (int)B, nullptr, nullptr, nullptr, nullptr};
-      const Proj sg = make_proj(a->shared_gate, (int)Is, (int)H), su = make_proj(a->shared_up, (int)Is, (int)H),
-                 sd = make_proj(a->shared_down, (int)H, (int)Is);
-      phases(sg, su, sd, dense, 1, (int)B, (int)Is, ws.sh_act, ws.sh_y, [](int) {});
+      shared_gate_up();
+      shared_down();
       if ((rc = check_launch("moe shared expert kernels"))) return rc;
     }
     DecArgs D;
@@ -1542,9 +1555,9 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     D.out = a->out;
     D.S = DecShared{};
     if (fused_shared) {
-      D.S.gate = make_proj(a->shared_gate, (int)Is, (int)H);
-      D.S.up = make_proj(a->shared_up, (int)Is, (int)H);
-      D.S.down = make_proj(a->shared_down, (int)H, (int)Is);
+      D.S.gate = sg;
+      D.S.up = su;
+      D.S.down = sd;
       D.S.is = (int)Is;
       D.S.act = ws.sh_act;
       D.S.y = ws.sh_y;
@@ -1615,6 +1628,9 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     set_error("moe_forward: prefill tile size mismatch");
     return Q6MOE_ERR_HIP;
   }
+  // the shared expert's items in the routed launches
+  const bool join_gu = sh_tiled_gu && tiled_gu, join_dn = sh_tiled_dn && tiled_dn;
+  if (Is && !join_gu) shared_gate_up();
   // gate/up + SwiGLU
   if (w8_gu) {
     mark(1);
@@ -1625,7 +1641,8 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     mark(2);
   } else if (tiled_gu) {
     // events[1] and [2] take the gate/up kernel's own start and end timestamps
-    launch_moe_prefill_gate_up(fmt, g, u, ws, max_tiles, a->x, (int)B, (int)H, (int)I, s,
+    const PfDense D = join_gu ? pf_dense_gate_up(sg, su, a->x, (int)B, ws.sh_act) : PfDense{};
+    launch_moe_prefill_gate_up(fmt, g, u, ws, max_tiles, a->x, (int)B, (int)H, (int)I, D, s,
                                a->events ? a->events[1] : nullptr, a->events ? a->events[2] : nullptr);
   } else {
     mark(1);
@@ -1641,20 +1658,15 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     launch_act_q8(ws.act, B * K, (int)I, ws.hdr + 1, aq, aq_s, s);  // rows beyond the routes are skipped
     launch_w8(false, d, d, routed, slots, 1, W8Src{aq, aq_s, (int)I}, ws.y, s);
   } else if (tiled_dn) {
-    launch_moe_prefill_down(fmt_dn, d, ws, max_tiles, (int)(B * K), (int)H, (int)I, s);
+    const PfDense D = join_dn ? pf_dense_down(sd, ws.sh_act, (int)B, ws.sh_y) : PfDense{};
+    launch_moe_prefill_down(fmt_dn, d, ws, max_tiles, (int)(B * K), (int)H, (int)I, D, s);
   } else {
     dispatch_format(fmt_dn, [&](auto fd) {
       launch_down<decltype(fd)::value>(d, routed, slots, max_tokens, ws.act, (int)H, (int)I, ws.y, s);
     });
   }
+  if (Is && !join_dn) shared_down();
   if ((rc = check_launch("moe expert kernels"))) return rc;
-  if (Is) {
-    TokenSrc dense{1, (int)B, nullptr, nullptr, nullptr, nullptr};
-    const Proj sg = make_proj(a->shared_gate, (int)Is, (int)H), su = make_proj(a->shared_up, (int)Is, (int)H),
-               sd = make_proj(a->shared_down, (int)H, (int)Is);
-    phases(sg, su, sd, dense, 1, (int)B, (int)Is, ws.sh_act, ws.sh_y, [](int) {});
-    if ((rc = check_launch("moe shared expert kernels"))) return rc;
-  }
   mark(3);
   hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)B, (unsigned)cdiv(H, 256 * 8)), dim3(256), 0, s,
                      ws.tok_pos, ws.route_w, ws.y, (int)K, (int)H, ws.sh_y, sh_scale, a->out);

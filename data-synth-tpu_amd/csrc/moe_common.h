@@ -207,11 +207,23 @@ int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStre
 bool pf_gate_up_supported(int fmt, int64_t H, int64_t I);
 bool pf_down_supported(int fmt, int64_t H, int64_t I);
 int64_t pf_tile_routes();
+// A dense expert (the always-on shared one: every token, weight 1) whose items
+// run in the tiled launches with the routed ones; tiles == 0: none. max_tiles
+// == 0 in the launches below: no routed items (``ws`` is then not read).
+struct PfDense {
+  Proj p0, p1;         // gate and up, or down (p0)
+  const uint16_t* in;  // x [tokens, H], or the activations [tokens, p0.k]
+  uint16_t* out;       // activations [tokens, rows], or the expert's output
+  int tokens, tiles;   // 128-token tiles
+  int ncol, rows;      // column blocks of output rows, output rows
+};
+PfDense pf_dense_gate_up(const Proj& g, const Proj& u, const uint16_t* x, int tokens, uint16_t* act);
+PfDense pf_dense_down(const Proj& d, const uint16_t* act, int tokens, uint16_t* y);
 int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles,
-                               const uint16_t* x, int B, int H, int I, hipStream_t s, void* gate_up_start,
-                               void* after_gate_up);
+                               const uint16_t* x, int B, int H, int I, const PfDense& D, hipStream_t s,
+                               void* gate_up_start, void* after_gate_up);
 int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I,
-                            hipStream_t s);
+                            const PfDense& D, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Unit decoders: 16 output rows x one 256-wide K block -> 8 MFMA A operands.

@@ -331,17 +331,40 @@ struct Tile {
   int r0, nv;  // first route position, valid routes (<= kM)
 };
 
-// Work item of workgroup blockIdx.x: (tile, column block), column block
-// fastest. Workgroup i runs on XCD i % 8 (round-robin dispatch), so the items
-// are split into eight contiguous runs, one per XCD, each walked in dispatch
-// order: the workgroups that share a token tile (its column blocks) or an
-// expert's weights (its tiles) run on one XCD at the same time and share its
-// L2. Returns false past the last item.
-__device__ __forceinline__ bool pf_item(const MoeWs& ws, int ncol, int& tile, int& col) {
+// Work item of workgroup blockIdx.x. Workgroup i runs on XCD i % 8
+// (round-robin dispatch), so the items are split into eight contiguous runs,
+// one per XCD, each walked in dispatch order.
+// The dense expert's items (D.ncol column blocks x D.tiles token tiles) come
+// first, an eighth on each XCD, since they are full tiles over the longest K;
+// token tile fastest: the workgroups that share a block of its weights run on
+// one XCD at the same time and share its L2 (every XCD reads the tokens, which
+// are the smaller side).
+// Routed items are (tile, column block), column block fastest: those that
+// share a token tile (its column blocks) or an expert's weights (its tiles)
+// run together. ncol 0: no routed items. Returns false past the last item.
+// kDense false: a launch without dense items, compiled apart (the choice per
+// item cost the routed-only 4096-token step 0.6 %).
+template <bool kDense>
+__device__ __forceinline__ bool pf_item(const MoeWs& ws, int ncol, const PfDense& D, bool& dense, int& tile, int& col) {
+  const int xcd = blockIdx.x & 7;
+  int k = blockIdx.x >> 3;
+  dense = false;
+  if constexpr (kDense) {
+    const int nd = D.tiles * D.ncol, rd = (nd + 7) >> 3;
+    dense = k < rd;
+    if (dense) {
+      const int item = xcd * rd + k;
+      if (item >= nd) return false;
+      col = item / D.tiles;
+      tile = item - col * D.tiles;
+      return true;
+    }
+    if (ncol == 0) return false;
+    k -= rd;
+  }
   const int ntiles = ws.hdr[2];
   const int items = ntiles * ncol;
   const int run = (items + 7) >> 3;
-  const int xcd = blockIdx.x & 7, k = blockIdx.x >> 3;
   const int item = xcd * run + k;
   if (k >= run || item >= items) return false;
   tile = item / ncol;
@@ -354,6 +377,17 @@ __device__ __forceinline__ void tile_info(const MoeWs& ws, int tile, Tile& T) {
   T.expert = d.expert;
   T.r0 = d.r0;
   T.nv = d.nv;
+}
+
+// The item's tile: the routing's record, or kM consecutive tokens.
+__device__ __forceinline__ void item_tile(const MoeWs& ws, const PfDense& D, bool dense, int tile, Tile& T) {
+  if (dense) {
+    T.expert = 0;
+    T.r0 = tile * kM;
+    T.nv = D.tokens - T.r0 < kM ? D.tokens - T.r0 : kM;
+  } else {
+    tile_info(ws, tile, T);
+  }
 }
 
 // Token rows of this wave's token-tile DMA: instruction i fills granules
@@ -524,29 +558,35 @@ __device__ __forceinline__ void with_column_groups(int nv, F&& f) {
 
 }  // namespace pf
 
-template <int FMT>
+template <int FMT, bool kDense>
 __global__ void __launch_bounds__(64 * pf::kWaves, 2)
     moe_pf_gate_up_kernel(Proj gate, Proj up, MoeWs ws, const uint16_t* __restrict__ x, int tokens, int hidden,
-                          uint16_t* __restrict__ act, int inter) {
+                          uint16_t* __restrict__ act_r, int inter_r, int ncol, PfDense D) {
   using namespace pf;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   Tile T;
+  bool dense;
   int tile, col;
-  if (!pf_item(ws, inter / (16 * kWaves), tile, col)) return;
-  tile_info(ws, tile, T);
+  if (!pf_item<kDense>(ws, ncol, D, dense, tile, col)) return;
+  item_tile(ws, D, dense, tile, T);
+  uint16_t* const act = dense ? D.out : act_r;
+  const int inter = dense ? D.rows : inter_r;
   const int wave = wave_id(), lane = threadIdx.x & 63;
   const int jA = lane >> 4, j = lane & 15;
   const int rgb = col * kWaves + wave;  // this wave's row group (gate and up)
   with_column_groups(T.nv, [&](auto ncg_c) {
     constexpr int NCG = decltype(ncg_c)::value;
-    const Proj projs[2] = {gate, up};
+    const Proj projs[2] = {dense ? D.p0 : gate, dense ? D.p1 : up};
     const int unit_proj[kUnits] = {0, 1};
     f32x4 acc[kUnits][NCG];
 #pragma unroll
     for (int u = 0; u < kUnits; ++u)
 #pragma unroll
       for (int t = 0; t < NCG; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto row_of = [&](int t) { return ws.route_tok[T.r0 + (t < T.nv ? t : T.nv - 1)]; };
+    auto row_of = [&](int t) {
+      const int r = T.r0 + (t < T.nv ? t : T.nv - 1);
+      return dense ? r : ws.route_tok[r];
+    };
     if (hidden % 256 == 0)
       pf_stream<FMT, NCG, true>(smem, projs, unit_proj, [&](int) { return rgb; }, x, tokens, row_of, hidden,
                                 T.expert, acc);
@@ -574,22 +614,26 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
   });
 }
 
-template <int FMT>
+template <int FMT, bool kDense>
 __global__ void __launch_bounds__(64 * pf::kWaves, 2)
-    moe_pf_down_kernel(Proj down, MoeWs ws, const uint16_t* __restrict__ act, int routes, int inter,
-                       uint16_t* __restrict__ y, int hidden) {
+    moe_pf_down_kernel(Proj down, MoeWs ws, const uint16_t* __restrict__ act_r, int routes, int inter_r,
+                       uint16_t* __restrict__ y_r, int hidden, int ncol, PfDense D) {
   using namespace pf;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   Tile T;
+  bool dense;
   int tile, col;
-  if (!pf_item(ws, hidden / (32 * kWaves), tile, col)) return;
-  tile_info(ws, tile, T);
+  if (!pf_item<kDense>(ws, ncol, D, dense, tile, col)) return;
+  item_tile(ws, D, dense, tile, T);
+  const uint16_t* const act = dense ? D.in : act_r;
+  uint16_t* const y = dense ? D.out : y_r;
+  const int inter = dense ? D.p0.k : inter_r, act_rows = dense ? D.tokens : routes;
   const int wave = wave_id(), lane = threadIdx.x & 63;
   const int jA = lane >> 4, j = lane & 15;
   const int rgb = col * 2 * kWaves + 2 * wave;  // this wave's two row groups
   with_column_groups(T.nv, [&](auto ncg_c) {
     constexpr int NCG = decltype(ncg_c)::value;
-    const Proj projs[1] = {down};
+    const Proj projs[1] = {dense ? D.p0 : down};
     const int unit_proj[kUnits] = {0, 0};
     f32x4 acc[kUnits][NCG];
 #pragma unroll
@@ -598,10 +642,10 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
       for (int t = 0; t < NCG; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto row_of = [&](int t) { return T.r0 + (t < T.nv ? t : T.nv - 1); };
     if (inter % 256 == 0)
-      pf_stream<FMT, NCG, true>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, routes, row_of, inter,
+      pf_stream<FMT, NCG, true>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
                                 T.expert, acc);
     else
-      pf_stream<FMT, NCG, false>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, routes, row_of, inter,
+      pf_stream<FMT, NCG, false>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
                                  T.expert, acc);
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) {
@@ -643,43 +687,76 @@ static void dispatch_pf_format(int fmt, F&& f) {
   }
 }
 
-static dim3 pf_grid(int ncol, int max_tiles) { return dim3((unsigned)(((int64_t)ncol * max_tiles + 7) / 8 * 8)); }
+// Workgroups: the dense items and the most routed items, each in eight equal runs.
+static dim3 pf_grid(int ncol, int max_tiles, const PfDense& D) {
+  const int64_t routed = ((int64_t)ncol * max_tiles + 7) / 8, dense = ((int64_t)D.tiles * D.ncol + 7) / 8;
+  return dim3((unsigned)(8 * (routed + dense)));
+}
+
+static int pf_tiles(int tokens) { return (tokens + pf::kM - 1) / pf::kM; }
+
+PfDense pf_dense_gate_up(const Proj& g, const Proj& u, const uint16_t* x, int tokens, uint16_t* act) {
+  return PfDense{g, u, x, act, tokens, pf_tiles(tokens), g.rows / (16 * pf::kWaves), g.rows};
+}
+PfDense pf_dense_down(const Proj& d, const uint16_t* act, int tokens, uint16_t* y) {
+  return PfDense{d, d, act, y, tokens, pf_tiles(tokens), d.rows / (32 * pf::kWaves), d.rows};
+}
+
+template <int FMT, bool kDense>
+static void pf_launch_gate_up(const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles, const uint16_t* x, int B,
+                              int H, int I, const PfDense& D, hipStream_t s, void* gate_up_start, void* after_gate_up) {
+  static std::atomic<uint64_t> attr_done{0};
+  once_per_device(attr_done, [] {
+    (void)hipFuncSetAttribute((const void*)moe_pf_gate_up_kernel<FMT, kDense>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds);
+  });
+  const int ncol = max_tiles ? I / (16 * pf::kWaves) : 0;
+  const dim3 grid = pf_grid(ncol, max_tiles, D), block(64 * pf::kWaves);
+  if (gate_up_start && after_gate_up) {
+    // the events take the kernel's own start and end timestamps
+    hipExtLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense>), grid, block, pf::kLds, s, (hipEvent_t)gate_up_start,
+                          (hipEvent_t)after_gate_up, 0, g, u, ws, x, B, H, ws.act, I, ncol, D);
+  } else {
+    hipLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense>), grid, block, pf::kLds, s, g, u, ws, x, B, H, ws.act, I,
+                       ncol, D);
+    if (after_gate_up) (void)hipEventRecord((hipEvent_t)after_gate_up, s);
+  }
+}
+
+template <int FMT, bool kDense>
+static void pf_launch_down(const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I, const PfDense& D,
+                           hipStream_t s) {
+  static std::atomic<uint64_t> attr_done{0};
+  once_per_device(attr_done, [] {
+    (void)hipFuncSetAttribute((const void*)moe_pf_down_kernel<FMT, kDense>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds);
+  });
+  const int ncol = max_tiles ? H / (32 * pf::kWaves) : 0;
+  hipLaunchKernelGGL((moe_pf_down_kernel<FMT, kDense>), pf_grid(ncol, max_tiles, D), dim3(64 * pf::kWaves), pf::kLds,
+                     s, d, ws, ws.act, routes, I, ws.y, H, ncol, D);
+}
 
 int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles,
-                               const uint16_t* x, int B, int H, int I, hipStream_t s, void* gate_up_start,
-                               void* after_gate_up) {
+                               const uint16_t* x, int B, int H, int I, const PfDense& D, hipStream_t s,
+                               void* gate_up_start, void* after_gate_up) {
   dispatch_pf_format(fmt, [&](auto fc) {
     constexpr int FMT = decltype(fc)::value;
-    static std::atomic<uint64_t> attr_done{0};
-    once_per_device(attr_done, [] {
-      (void)hipFuncSetAttribute((const void*)moe_pf_gate_up_kernel<FMT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                pf::kLds);
-    });
-    const dim3 grid = pf_grid(I / (16 * pf::kWaves), max_tiles);
-    if (gate_up_start && after_gate_up) {
-      // the events take the kernel's own start and end timestamps
-      hipExtLaunchKernelGGL(moe_pf_gate_up_kernel<FMT>, grid, dim3(64 * pf::kWaves), pf::kLds, s,
-                            (hipEvent_t)gate_up_start, (hipEvent_t)after_gate_up, 0, g, u, ws, x, B, H, ws.act, I);
-    } else {
-      hipLaunchKernelGGL(moe_pf_gate_up_kernel<FMT>, grid, dim3(64 * pf::kWaves), pf::kLds, s, g, u, ws, x, B, H,
-                         ws.act, I);
-      if (after_gate_up) (void)hipEventRecord((hipEvent_t)after_gate_up, s);
-    }
+    if (D.tiles)
+      pf_launch_gate_up<FMT, true>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
+    else
+      pf_launch_gate_up<FMT, false>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
   });
   return Q6MOE_OK;
 }
 
 int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I,
-                            hipStream_t s) {
+                            const PfDense& D, hipStream_t s) {
   dispatch_pf_format(fmt, [&](auto fc) {
     constexpr int FMT = decltype(fc)::value;
-    static std::atomic<uint64_t> attr_done{0};
-    once_per_device(attr_done, [] {
-      (void)hipFuncSetAttribute((const void*)moe_pf_down_kernel<FMT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                pf::kLds);
-    });
-    hipLaunchKernelGGL(moe_pf_down_kernel<FMT>, pf_grid(H / (32 * pf::kWaves), max_tiles), dim3(64 * pf::kWaves),
-                       pf::kLds, s, d, ws, ws.act, routes, I, ws.y, H);
+    if (D.tiles)
+      pf_launch_down<FMT, true>(d, ws, max_tiles, routes, H, I, D, s);
+    else
+      pf_launch_down<FMT, false>(d, ws, max_tiles, routes, H, I, D, s);
   });
   return Q6MOE_OK;
 }

@@ -551,3 +551,23 @@ def test_largest_layer_every_family(device, largest_layer, tokens):
     want = oracle_moe.expert_ffn(L["gate"], L["up"], L["down"], L["x"][rows], L["ids"][rows], L["weights"][rows],
                                  types=("Q6_K", "Q6_K", "Q8_0"), hidden=256, intermediate=256, workers=8)
     assert_moe_close(outs[0], want)
+
+
+@pytest.mark.parametrize("qtype,down,shared,tokens,mode,inter", [
+    ("Q4_K", "Q4_K", 512, 65, 0, 256),     # joins the routed launches, a partial second 64 tokens
+    ("Q6_K", "Q6_K", 256, 128, 2, 256),    # one full tile
+    ("Q6_K", "Q8_0", 640, 129, 2, 256),    # a one-token second tile, K halves
+    ("Q5_K", "Q5_K", 256, 300, 2, 256),    # three tiles
+    ("Q8_0", "Q5_1", 64, 100, 2, 256),     # gate/up tiled, down's K of 64 on the generic kernel
+    ("Q8_0", "Q8_0", 96, 100, 2, 256),     # neither tiled
+    ("Q8_0", "Q8_0", 256, 100, 2, 96),     # tiled, the routed experts are not
+    ("Q4_K", "Q4_K", 512, 70, 1, 256),     # beside the decode launches, past their own 64 tokens
+    ("Q4_K", "Q4_K", 256, 3, 2, 256),      # fewer tokens than a column group
+])
+def test_shared_expert_of_many_tokens(device, qtype, down, shared, tokens, mode, inter):
+    L = moe_layer(seed=tokens + shared, experts=6, top_k=2, hidden=512, intermediate=inter, tokens=tokens,
+                  qtype=qtype, down_qtype=down, shared_intermediate=shared, pack=False)
+    got, ctx = _run(L, device, mode=mode, shared=L["shared"])
+    assert_moe_close(got, _oracle(L, shared=L["shared"]))
+    fn, tabs, x, ids, w, sh = ctx
+    np.testing.assert_array_equal(got, fn(*tabs, x, ids, w, shared=sh).float().cpu().numpy())
