@@ -984,13 +984,6 @@ __global__ void __launch_bounds__(256)
   scales[gid] = sc;
 }
 
-// Quantised activations: codes [rows, k] and scales [rows, k / 32].
-struct W8Src {
-  const int8_t* codes;
-  const float* scales;
-  int k;
-};
-
 __device__ __forceinline__ i32x4 mfma_i8(uint64_t a, uint64_t b, i32x4 c) {
   return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)a, (long)b, c, 0, 0, 0);
 }
@@ -1631,13 +1624,23 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   // the shared expert's items in the routed launches
   const bool join_gu = sh_tiled_gu && tiled_gu, join_dn = sh_tiled_dn && tiled_dn;
   if (Is && !join_gu) shared_gate_up();
+  // W8A8: tiled unless the items (active experts x column blocks) would leave
+  // the chip idle and no expert has more than a 64-token tile; there the kernel
+  // that splits K over 8 waves has more waves in flight. 128-expert top-8 layer
+  // (H 2048, I 768), step: 1 token 43.0 us split and 47.8 tiled, 2 tokens 49.1
+  // and 53.3, 8 tokens 124 and 85.7, 40 tokens 227 and 144, 1024 tokens 2436 and 295.
+  const auto w8_tiled = [&](int64_t cols) { return slots * cols >= 512 || B * K > 64 * slots; };
   // gate/up + SwiGLU
   if (w8_gu) {
     mark(1);
     int8_t* xq = reinterpret_cast<int8_t*>(w + L.xq);
     float* xq_s = reinterpret_cast<float*>(w + L.xq_s);
     launch_act_q8(a->x, B, (int)H, nullptr, xq, xq_s, s);
-    launch_w8(true, g, u, routed, slots, 0, W8Src{xq, xq_s, (int)H}, ws.act, s);
+    const W8Src src{xq, xq_s, (int)H};
+    if (rows32 && w8_tiled(I / 64) && pf_w8_supported(true, I, H))
+      launch_moe_prefill_w8(true, g, u, ws, max_tiles, 0, src, (int)B, ws.act, s);
+    else
+      launch_w8(true, g, u, routed, slots, 0, src, ws.act, s);
     mark(2);
   } else if (tiled_gu) {
     // events[1] and [2] take the gate/up kernel's own start and end timestamps
@@ -1656,7 +1659,11 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     int8_t* aq = reinterpret_cast<int8_t*>(w + L.aq);
     float* aq_s = reinterpret_cast<float*>(w + L.aq_s);
     launch_act_q8(ws.act, B * K, (int)I, ws.hdr + 1, aq, aq_s, s);  // rows beyond the routes are skipped
-    launch_w8(false, d, d, routed, slots, 1, W8Src{aq, aq_s, (int)I}, ws.y, s);
+    const W8Src src{aq, aq_s, (int)I};
+    if (rows32 && w8_tiled(H / 128) && pf_w8_supported(false, H, I))
+      launch_moe_prefill_w8(false, d, d, ws, max_tiles, 1, src, (int)(B * K), ws.y, s);
+    else
+      launch_w8(false, d, d, routed, slots, 1, src, ws.y, s);
   } else if (tiled_dn) {
     const PfDense D = join_dn ? pf_dense_down(sd, ws.sh_act, (int)B, ws.sh_y) : PfDense{};
     launch_moe_prefill_down(fmt_dn, d, ws, max_tiles, (int)(B * K), (int)H, (int)I, D, s);
@@ -1721,7 +1728,16 @@ extern "C" int q6moe_q8_matmul(const uint16_t* x, int64_t m, int64_t k, const ui
   launch_act_q8(x, m, (int)k, nullptr, codes, scales, s);
   q6moe_table t{Q6MOE_Q8_0, table, (int64_t)unit_table_bytes(Q6MOE_Q8_0, n, k), nullptr, 0};
   const Proj p = make_proj(t, (int)n, (int)k);
-  TokenSrc dense{1, (int)m, nullptr, nullptr, nullptr, nullptr};
-  launch_w8(false, p, p, dense, 1, 0, W8Src{codes, scales, (int)k}, y, s);
+  const W8Src src{codes, scales, (int)k};
+  // Tiled above 64 tokens (64-token tiles, no K split); below, splitting K over
+  // 8 waves gives the few row groups more waves. 4096 x 4096: 64 tokens 46.7 us
+  // split, 59.5 tiled; 128 tokens 88.9 and 60.4; 640 x 2560: 35.5 and 37.7, 66.0
+  // and 37.9.
+  if (m > 64 && m * k < (1ll << 31) && aligned(y, 8) && pf_w8_supported(false, n, k)) {
+    launch_prefill_w8_dense(p, src, (int)m, y, s);
+  } else {
+    TokenSrc dense{1, (int)m, nullptr, nullptr, nullptr, nullptr};
+    launch_w8(false, p, p, dense, 1, 0, src, y, s);
+  }
   return check_launch("q8_matmul kernels");
 }

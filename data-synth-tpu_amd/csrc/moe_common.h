@@ -225,6 +225,23 @@ int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeW
 int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I,
                             const PfDense& D, hipStream_t s);
 
+// W8A8 policy: quantised activations, codes [rows, k] and scales [rows, k / 32].
+struct W8Src {
+  const int8_t* codes;
+  const float* scales;
+  int k;
+};
+
+// The tiled W8A8 projections of Q8_0 tables (pair: gate and up with the SwiGLU
+// epilogue; otherwise one projection): K a multiple of 128, rows of 64 (pair)
+// or 128, and activations within 32-bit byte offsets. ``route_rows``: the
+// activation rows are route positions (down), not tokens. The dense form takes
+// tokens 0.. of one table.
+bool pf_w8_supported(bool pair, int64_t rows, int64_t k);
+void launch_moe_prefill_w8(bool pair, const Proj& p0, const Proj& p1, const MoeWs& ws, int max_tiles, int route_rows,
+                           const W8Src& a, int a_rows, uint16_t* out, hipStream_t s);
+void launch_prefill_w8_dense(const Proj& p, const W8Src& a, int tokens, uint16_t* out, hipStream_t s);
+
 // ---------------------------------------------------------------------------
 // Unit decoders: 16 output rows x one 256-wide K block -> 8 MFMA A operands.
 // ---------------------------------------------------------------------------

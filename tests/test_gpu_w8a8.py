@@ -121,3 +121,45 @@ def test_int8_q8_policy_matches_oracle(device, qtype, tokens, mode):
     bf16 = oracle_moe.expert_ffn(L["gate"], L["up"], L["down"], L["x"], L["ids"], L["weights"],
                                  types=(qtype, qtype, "Q8_0"), hidden=512, intermediate=256)
     assert not np.array_equal(want, bf16)  # the policy changes the arithmetic
+
+
+@pytest.mark.parametrize("m,k,n", [(65, 128, 128), (128, 640, 256), (129, 256, 128), (200, 384, 384)])
+def test_q8_matmul_tiled_shapes(device, m, k, n):
+    # above 64 tokens: 64-token tiles (one token past a tile, both halves of a
+    # 128-token tile), K of whole and half 256-wide blocks. A row of infinities
+    # follows row 5, whose last half block reads past its end.
+    rng = np.random.default_rng(m + k + n)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    x[0] = 0
+    raw = pack_q8(rng.normal(0, 0.05, (n, k)).astype(np.float32))
+    token = torch.from_numpy(x).to(device).to(torch.bfloat16)
+    packed = torch.from_numpy(raw).to(device)
+    got = q8_matmul(token, packed).float().cpu().numpy()
+    want = bf16_round(oracle_compute.q8_matmul(token.float().cpu().numpy(), raw))
+    assert_moe_close(got, want, ref_gate=False)
+    np.testing.assert_array_equal(got[0], 0)
+    token[6] = float("inf")
+    again = q8_matmul(token, packed).float().cpu().numpy()
+    np.testing.assert_array_equal(np.delete(again, 6, 0), np.delete(got, 6, 0))
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 128), (384, 640)])
+def test_int8_q8_tiles_of_every_width(device, hidden, inter):
+    # Top-1 routes assigned so that the experts hold every count of 16-route
+    # column groups, full 64-route parts and one-route tails; K of odd halves.
+    counts = [1, 15, 16, 17, 32, 33, 48, 64, 65, 127, 128, 129, 200]
+    experts, tokens = len(counts), sum(counts)
+    L = moe_layer(seed=17, experts=experts, top_k=1, hidden=hidden, intermediate=inter, tokens=tokens, qtype="Q8_0",
+                  down_qtype="Q8_0", pack=False)
+    ids = np.random.default_rng(3).permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    fn = expert_parallel(None, gate_type="Q8_0", up_type="Q8_0", down_type="Q8_0", hidden=hidden,
+                         intermediate=inter, compute="int8_q8")
+    tabs = fn.prepare(*(L[n].reshape(experts, -1) for n in ("gate", "up", "down")), device)
+    x = torch.from_numpy(L["x"]).to(device).to(torch.bfloat16)
+    w = torch.from_numpy(L["weights"]).to(device).to(torch.bfloat16)
+    args = (*tabs, x, torch.from_numpy(ids).to(device), w)
+    got = fn(*args).float().cpu().numpy()
+    want = oracle_moe.expert_ffn(L["gate"], L["up"], L["down"], L["x"], ids, L["weights"], types=("Q8_0",) * 3,
+                                 hidden=hidden, intermediate=inter, policy="int8_q8")
+    assert_moe_close(got, want)
+    np.testing.assert_array_equal(got, fn(*args).float().cpu().numpy())
