@@ -243,3 +243,27 @@ def test_dequantize_rows_hip_staged_and_fallback_paths(device, qtype):
         shifted = buf[1:].view(rows, nb, size)  # 1-byte offset: the byte path
         got = dequantize_rows(shifted, qtype, width, dtype=torch.bfloat16)
         np.testing.assert_array_equal(_bf16_bits(got), packed_q6.bf16_bits(want))
+
+
+@pytest.mark.parametrize("batch,outputs,inputs", [
+    (17, 130, 520), (17, 3, 8), (40, 64, 768), (64, 64, 256), (65, 67, 1544), (127, 320, 2560), (128, 65, 1408),
+    (200, 96, 3080), (64, 16448, 256)])
+def test_tiled_projection(device, batch, outputs, inputs):
+    # 64-token tiles from 64 tokens on (17 with up to three K blocks): one token
+    # past a tile, rows past the matrix, K ending inside a 128-wide half, K sets of
+    # unequal (or no) blocks, two and four sets. x is a view of wider rows whose
+    # padding must not enter.
+    raw = packed_q6.fixture(outputs, inputs)
+    wide = np.full((batch, inputs + 24), np.nan, np.float32)
+    x = wide[:, :inputs]
+    x[:] = np.random.default_rng(batch).normal(size=(batch, inputs))
+    x[0] = 0
+    data, scales = _to_dev(pack_q6(raw, inputs), device)
+    xt = torch.from_numpy(wide).to(device).to(torch.bfloat16)[:, :inputs]
+    got = q6_matmul(xt, data, scales, output_features=outputs)
+    want = packed_q6.projection_reference(x, raw)
+    np.testing.assert_allclose(got.cpu().numpy(), want, rtol=2e-5, atol=2e-4)
+    assert torch.all(got[0] == 0)
+    assert torch.equal(got, q6_matmul(xt.contiguous(), data, scales, output_features=outputs))
+    half = q6_matmul(xt, data, scales, output_features=outputs, out_dtype=torch.bfloat16)
+    assert torch.equal(half, got.to(torch.bfloat16))
