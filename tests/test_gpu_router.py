@@ -44,3 +44,21 @@ def test_router_ties_pick_the_lower_id(device):
 def test_router_rejects_more_than_1024_experts(device):
     with pytest.raises(ValueError, match="experts <= 1024"):
         routes(torch.zeros((2, 1025), device=device), 4)
+
+
+@pytest.mark.parametrize("experts", [64, 128, 129, 300, 512, 513, 1024])
+def test_router_slot_counts_and_ties(device, experts):
+    # every number of logits per lane, at its first and last width, with ties
+    # across lanes, within a lane (ids 64 apart) and across rows of 16 lanes
+    rng = np.random.default_rng(experts)
+    logits = rng.standard_normal((9, experts)).astype(np.float32)
+    logits[1] = 0.25
+    logits[2, rng.permutation(experts)[:20]] = 5.0
+    logits[3, ::64] = 4.0
+    logits[4, 1::16] = 4.0
+    logits[5] = np.round(logits[5])
+    k = min(experts, 32)
+    ids, w = routes(torch.from_numpy(logits).to(device), k)
+    want_ids, want_w = oracle_routing.route(logits, k)
+    np.testing.assert_array_equal(ids.cpu().numpy(), want_ids)
+    np.testing.assert_allclose(w.float().cpu().numpy(), want_w, rtol=2 ** -7, atol=0)
