@@ -180,14 +180,24 @@ __device__ __forceinline__ void route_merge(const int* s_ids, float* s_w, int* c
   }
 }
 
+// The workgroups from ``first`` on compute the shared expert's gate, one token
+// per wave. Returns whether this workgroup is one of them.
+__device__ __forceinline__ bool gate_block(const SharedGate& g, int first) {
+  if ((int)blockIdx.x < first) return false;
+  const int b = ((int)blockIdx.x - first) * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (b < g.tokens) shared_gate_token(g, b, threadIdx.x & 63);
+  return true;
+}
+
 // Routing, pass 1 (one workgroup per chunk of kChunk tokens, one lane per
 // token): merged BF16 weight of each first occurrence of an id in a token
 // (experts.py:66-73; 0 for repeats and out-of-range ids) and the chunk's
 // route count per expert.
 __global__ void __launch_bounds__(kChunk)
     moe_route_count_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K,
-                           int E, MoeWs ws, int* __restrict__ chunk_cnt) {
+                           int E, int nchunks, MoeWs ws, int* __restrict__ chunk_cnt, SharedGate gate) {
   extern __shared__ int sm[];
+  if (gate_block(gate, nchunks)) return;
   int* s_ids = sm;                                            // [kChunk * K]
   float* s_w = reinterpret_cast<float*>(sm + kChunk * K);     // [kChunk * K] weights, then merged weights
   __shared__ int cnt[kMaxExperts];
@@ -441,8 +451,9 @@ __global__ void __launch_bounds__(kMaxExperts)
 // each expert are 0). Same outputs as the three launches.
 __global__ void __launch_bounds__(kMaxExperts)
     moe_route_small_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K, int E,
-                           int mtile, MoeWs ws) {
+                           int mtile, MoeWs ws, SharedGate gate) {
   extern __shared__ int sm[];
+  if (gate_block(gate, 1)) return;
   int* s_ids = sm;                                                     // [kChunk * K]
   float* s_w = reinterpret_cast<float*>(sm + kChunk * K);              // [kChunk * K] staged weights
   float* s_m = reinterpret_cast<float*>(sm + 2 * kChunk * K);          // [kChunk * K] merged weights
@@ -775,31 +786,9 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<u32x4*>(out + (int64_t)b * hidden + h) = o;
 }
 
-// Shared-expert gate (kaggle/qwen38_tpu/math.py:283 with linear and sigmoid of
-// math.py:10-24): gate[b] = RNE(sigmoid(RNE(x[b] . w))), x BF16 [B, H], w BF16
-// [H], FP32 accumulation. One wave per token; lane l sums the products of
-// columns 8(l + 64i) .. +7 in column order, then the 64 lane sums meet in a
-// fixed butterfly, so the result does not depend on scheduling.
-__global__ void __launch_bounds__(64)
-    moe_shared_gate_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, int hidden,
-                           uint16_t* __restrict__ gate) {
-  const int b = blockIdx.x, lane = threadIdx.x;
-  const uint16_t* xr = x + (int64_t)b * hidden;
-  float acc = 0.f;
-  for (int h = 8 * lane; h < hidden; h += 512) {
-    const u32x4 xv = *reinterpret_cast<const u32x4*>(xr + h);
-    const u32x4 wv = *reinterpret_cast<const u32x4*>(w + h);
-#pragma unroll
-    for (int q = 0; q < 8; ++q)
-      acc += bf16_to_float((uint16_t)(xv[q >> 1] >> (16 * (q & 1)))) *
-             bf16_to_float((uint16_t)(wv[q >> 1] >> (16 * (q & 1))));
-  }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) acc += __shfl_xor(acc, off);
-  if (lane == 0) {
-    const float g = bf16_round(acc);
-    gate[b] = bf16_bits(sigmoid_acc(g));
-  }
+// The shared expert's gate of many tokens beside the decode-step launches.
+__global__ void __launch_bounds__(64) moe_shared_gate_kernel(SharedGate g) {
+  shared_gate_token(g, blockIdx.x, threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1471,13 +1460,13 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   ws.sh_y = Is ? reinterpret_cast<uint16_t*>(w + L.sh_y) : nullptr;
 
   hipStream_t s = (hipStream_t)stream;
-  // Per-token shared-expert gate: the caller's, or computed here from the router.
+  // Per-token shared-expert gate: the caller's, or computed here from the router
+  // in the first launch of the path.
   const uint16_t* sh_scale = a->shared_scale;
+  SharedGate gate{};
   if (Is && a->shared_router) {
-    uint16_t* g = reinterpret_cast<uint16_t*>(w + L.sh_gate);
-    hipLaunchKernelGGL(moe_shared_gate_kernel, dim3((unsigned)B), dim3(64), 0, s, a->x, a->shared_router, (int)H, g);
-    if ((rc = check_launch("moe_shared_gate_kernel"))) return rc;
-    sh_scale = g;
+    gate = SharedGate{a->x, a->shared_router, reinterpret_cast<uint16_t*>(w + L.sh_gate), (int)H, (int)B};
+    sh_scale = gate.gate;
   }
   auto mark = [&](int i) {
     if (a->events && a->events[i]) (void)hipEventRecord((hipEvent_t)a->events[i], s);
@@ -1520,6 +1509,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     // up to kDecSharedTokens tokens the shared expert runs inside the decode launches
     const bool fused_shared = Is && B <= kDecSharedTokens;
     if (Is && !fused_shared) {
+      if (gate.tokens) hipLaunchKernelGGL(moe_shared_gate_kernel, dim3((unsigned)B), dim3(64), 0, s, gate);
       shared_gate_up();
       shared_down();
       if ((rc = check_launch("moe shared expert kernels"))) return rc;
@@ -1554,6 +1544,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
       D.S.is = (int)Is;
       D.S.act = ws.sh_act;
       D.S.y = ws.sh_y;
+      D.S.gate_of = gate;
     }
     // events[1] and [2] take the gate/up kernel's own start and end timestamps
     D.gate_up_start = a->events ? a->events[1] : nullptr;
@@ -1585,11 +1576,13 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     if (nchunks == 1) {
       // one chunk: the three passes in one launch (its counts and positions in LDS)
       const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);
-      hipLaunchKernelGGL(moe_route_small_kernel, dim3(1), dim3(lanes), scatter_lds(K, E) + (size_t)E * 4, s, a->ids,
-                         a->weights, (int)B, (int)K, (int)E, (int)kPrefillTile, ws);
+      const dim3 grid(1 + (unsigned)cdiv(gate.tokens, lanes / 64));
+      hipLaunchKernelGGL(moe_route_small_kernel, grid, dim3(lanes), scatter_lds(K, E) + (size_t)E * 4, s, a->ids,
+                         a->weights, (int)B, (int)K, (int)E, (int)kPrefillTile, ws, gate);
     } else {
-      hipLaunchKernelGGL(moe_route_count_kernel, dim3(nchunks), dim3(kChunk), (size_t)kChunk * K * 8, s, a->ids,
-                         a->weights, (int)B, (int)K, (int)E, ws, chunk_cnt);
+      const dim3 grid((unsigned)(nchunks + cdiv(gate.tokens, kChunk / 64)));
+      hipLaunchKernelGGL(moe_route_count_kernel, grid, dim3(kChunk), (size_t)kChunk * K * 8, s, a->ids, a->weights,
+                         (int)B, (int)K, (int)E, nchunks, ws, chunk_cnt, gate);
       if (nchunks <= kFoldChunks) {
         // the scan folded into the scatter workgroups (up to 8192 tokens)
         const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);

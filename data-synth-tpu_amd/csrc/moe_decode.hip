@@ -804,7 +804,8 @@ __device__ __forceinline__ void dec_gate_up_item(uint8_t* smem, uint8_t* ring, i
 }
 
 // Items: the shared expert's (row group, pass of 16 tokens) first (sh.is > 0),
-// then (row group, expert slot) with the row group fastest.
+// then its gate, one token each, then (row group, expert slot) with the row
+// group fastest.
 template <int FMT, bool kFullK>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
     moe_dec_gate_up_kernel(Proj gate, Proj up, DecRoute R, DecTables T, const uint16_t* __restrict__ x,
@@ -828,8 +829,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
                                   sh.is);
     return;
   }
+  const int first = sh_items + sh.gate_of.tokens;
+  if (item < first) {
+    if (wave == 0) shared_gate_token(sh.gate_of, item - sh_items, threadIdx.x & 63);
+    return;
+  }
   const int groups_i = (inter + 15) / 16;
-  const int rg = (item - sh_items) % groups_i, slot = (item - sh_items) / groups_i;
+  const int rg = (item - first) % groups_i, slot = (item - first) / groups_i;
   SlotRoute sr;
   if (!dec_route(R, slot, rg == 0 && wave == 0, T, ring, tok, sr)) return;
   dec_gate_up_item<FMT, kFullK>(smem, ring, wl, gate, up, sr.expert, rg, sr.t0, sr.cnt, tok, x, R.B, hidden, act,
@@ -1120,6 +1126,7 @@ static int launch(const DecArgs& A, hipStream_t s) {
   // 64 entries that every wave repeats cheaply
   const int kb_i = (int)cdiv(A.I, kQK);
   const bool long_dn = kb_i % 2 == 0 && kb_i >= 4 && A.R.B * A.R.K <= 64;
+  const unsigned grid_gu = (unsigned)(items_gu + (A.S.is ? A.S.gate_of.tokens : 0));
   const int ns_gu = split_for(items_gu, false), ns_dn = split_for(items_dn, long_dn);
   // One launch for gate/up and down where the routes are spread thin (fewer
   // than 0.4 routes per expert on average: most active experts see one route,
@@ -1153,11 +1160,11 @@ static int launch(const DecArgs& A, hipStream_t s) {
   } else {
     if (A.gate_up_start && A.after_gate_up) {
       // the events take the kernel's own start and end timestamps
-      hipExtLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3((unsigned)items_gu), dim3(64 * ns_gu),
+      hipExtLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3(grid_gu), dim3(64 * ns_gu),
                             ns_gu * lds_gu, s, (hipEvent_t)A.gate_up_start, (hipEvent_t)A.after_gate_up, 0, A.gate,
                             A.up, A.R, A.T, A.x, A.H, A.act, A.I, A.S);
     } else {
-      hipLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3((unsigned)items_gu), dim3(64 * ns_gu),
+      hipLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3(grid_gu), dim3(64 * ns_gu),
                          ns_gu * lds_gu, s, A.gate, A.up, A.R, A.T, A.x, A.H, A.act, A.I, A.S);
       if (A.after_gate_up) (void)hipEventRecord((hipEvent_t)A.after_gate_up, s);
     }

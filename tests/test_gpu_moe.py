@@ -571,3 +571,20 @@ def test_shared_expert_of_many_tokens(device, qtype, down, shared, tokens, mode,
     assert_moe_close(got, _oracle(L, shared=L["shared"]))
     fn, tabs, x, ids, w, sh = ctx
     np.testing.assert_array_equal(got, fn(*tabs, x, ids, w, shared=sh).float().cpu().numpy())
+
+
+@pytest.mark.parametrize("tokens,mode", [(1, 1), (17, 1), (64, 1), (65, 1), (1, 2), (65, 2), (256, 2), (257, 2)])
+def test_shared_gate_of_every_path(device, tokens, mode):
+    # The gate's waves ride in the decode gate/up launch, in the one-launch and
+    # the chunked routing, and run alone beside the decode launches past 64
+    # tokens. One-hot router and scaled tokens: gate = RNE(sigmoid(x[b, 3])).
+    L = moe_layer(seed=tokens, experts=6, top_k=2, hidden=512, intermediate=256, tokens=tokens,
+                  shared_intermediate=256, pack=False)
+    _, (fn, tabs, x, ids, w, sh) = _run(L, device, mode=mode, shared=L["shared"])
+    router = torch.zeros(512, device=device, dtype=torch.bfloat16)
+    router[3] = 1
+    got = fn(*tabs, x, ids, w, shared=dict(sh, router=router))
+    scale = torch.sigmoid(x[:, 3].float().cpu().double()).to(torch.float32).to(torch.bfloat16).to(device)
+    want = fn(*tabs, x, ids, w, shared=dict(sh, scale=scale))
+    assert (got == want).float().mean() > 0.99  # a sigmoid an ulp off may round its token's gate the other way
+    np.testing.assert_allclose(got.float().cpu().numpy(), want.float().cpu().numpy(), rtol=1e-2, atol=1e-2)
