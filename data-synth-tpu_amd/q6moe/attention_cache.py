@@ -16,10 +16,11 @@ with the reference contract and error messages.
 """
 
 import ctypes
+from functools import lru_cache
 
 import torch
 
-from . import _lib
+from . import _launch, _lib
 
 
 def _dtype_code(dtype):
@@ -31,10 +32,24 @@ def _dtype_code(dtype):
 
 
 def _run(args, device):
-    lib = _lib.load()
-    with torch.cuda.device(device):
-        rc = lib.q6moe_kv_read(ctypes.byref(args), _lib.stream_handle(device))
-    _lib.check(rc, "kv_read")
+    _launch.run("kv_read", _lib.load().q6moe_kv_read, device, ctypes.byref(args))
+
+
+def _int32(t, device):
+    """``t`` as a contiguous int32 tensor on ``device`` (itself, usually)."""
+    if t.dtype is not torch.int32 or t.device != device:
+        t = t.to(device=device, dtype=torch.int32)
+    return t.contiguous()
+
+
+def _row_values(t):
+    """Values of a [pages, page_size, ...] tensor's [0, 0] (IndexError without one)."""
+    if t.ndim < 2 or not t.shape[0] or not t.shape[1]:
+        return t[0, 0].numel()
+    n = 1
+    for s in t.shape[2:]:
+        n *= s
+    return n
 
 
 def _group_of(c):
@@ -53,18 +68,15 @@ def quantize(x, group, scale_dtype=torch.bfloat16):
     rows, chans = xx.numel() // x.shape[-1], x.shape[-1]
     codes = torch.empty(x.shape, dtype=torch.int8, device=x.device)
     scale = torch.empty((*x.shape[:-1], chans // group), dtype=scale_dtype, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        rc = lib.q6moe_kv_quantize(xx.data_ptr(), _dtype_code(xx.dtype), rows, chans, group, codes.data_ptr(),
-                                   scale.data_ptr(), _dtype_code(scale_dtype), _lib.stream_handle(x.device))
-    _lib.check(rc, "kv_quantize")
+    _launch.run("kv_quantize", _lib.load().q6moe_kv_quantize, x.device, xx.data_ptr(), _dtype_code(xx.dtype), rows, chans,
+                group, codes.data_ptr(), scale.data_ptr(), _dtype_code(scale_dtype))
     return codes, scale
 
 
 def _write(x, codes, scales, *, layout, indices, active, batch, capacity, heads, dim, group, table=None,
            pool_pages=0, pages_per_seq=0, page_size=0):
     xx = x.reshape(batch, heads * dim).contiguous()
-    idx = indices.to(device=codes.device, dtype=torch.int32).contiguous()
+    idx = _int32(indices, codes.device)
     if idx.numel() != batch:
         raise ValueError("indices must hold one token slot per row")
     act = None
@@ -80,10 +92,7 @@ def _write(x, codes, scales, *, layout, indices, active, batch, capacity, heads,
     a.active = None if act is None else act.data_ptr()
     a.batch, a.capacity = batch, capacity
     a.kv_heads, a.head_dim, a.group = heads, dim, group
-    lib = _lib.load()
-    with torch.cuda.device(codes.device):
-        rc = lib.q6moe_kv_write(ctypes.byref(a), _lib.stream_handle(codes.device))
-    _lib.check(rc, "kv_write")
+    _launch.run("kv_write", _lib.load().q6moe_kv_write, codes.device, ctypes.byref(a))
 
 
 def write_quantized(cache, key, value, indices, active, c):
@@ -114,7 +123,7 @@ def write_paged(pool, scales, page_table, x, indices, *, page_size, kv_heads, he
     group = head_dim if group is None else group
     if pool.dtype != torch.int8 or pool.ndim < 3 or pool.shape[1] != page_size or not pool.is_contiguous():
         raise ValueError("pool must be contiguous int8 [pages, page_size, ...]")
-    table = page_table.to(device=pool.device, dtype=torch.int32).contiguous()
+    table = _int32(page_table, pool.device)
     batch, pps = table.shape
     _write(x, pool, scales, layout=1, indices=indices, active=active, batch=batch, capacity=pps * page_size,
            heads=kv_heads, dim=head_dim, group=group, table=table, pool_pages=pool.shape[0],
@@ -144,7 +153,7 @@ def read_quantized(cache, name, indices, c, dtype=torch.bfloat16, *, scale_gathe
         raise ValueError("indices and the scale plane must match the cache's batch and time")
     if plane.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError("scale plane must be BF16 or FP32")
-    idx = indices.to(device=codes.device, dtype=torch.int32).contiguous()
+    idx = _int32(indices, codes.device)
     out = torch.empty((batch, idx.shape[1], heads, dim), dtype=dtype, device=codes.device)
     codes, plane = codes.contiguous(), plane.contiguous()
     a = _lib.KvArgs()
@@ -171,14 +180,14 @@ def read_paged(pool, scales, page_table, *, page_size, kv_heads, head_dim, group
     if pool.dtype != torch.int8 or pool.ndim < 3 or pool.shape[1] != page_size:
         raise ValueError("pool must be int8 [pages, page_size, ...]")
     chans = kv_heads * head_dim
-    if pool[0, 0].numel() != chans:
+    if _row_values(pool) != chans:
         raise ValueError("pool rows must hold kv_heads * head_dim codes")
-    if scales[0, 0].numel() != chans // group:
+    if _row_values(scales) != chans // group:
         raise ValueError("scales must hold kv_heads * head_dim / group values per token")
-    table = page_table.to(device=pool.device, dtype=torch.int32).contiguous()
+    table = _int32(page_table, pool.device)
     batch, pps = table.shape
     cap = pps * page_size
-    idx = None if indices is None else indices.to(device=pool.device, dtype=torch.int32).contiguous()
+    idx = None if indices is None else _int32(indices, pool.device)
     sel = cap if idx is None else idx.shape[1]
     if out is None:
         out = torch.empty((batch, sel, kv_heads, head_dim), dtype=dtype, device=pool.device)
@@ -202,6 +211,11 @@ def read_paged(pool, scales, page_table, *, page_size, kv_heads, head_dim, group
     return out
 
 
+@lru_cache(maxsize=256)
+def _attn_workspace_bytes(batch, hq, kv_heads, pps, page_size):
+    return int(_lib.load().q6moe_attn_workspace_size(batch, hq, kv_heads, pps, page_size))
+
+
 def paged_decode_attention(q, k_pool, k_scales, v_pool, v_scales, page_table, lengths, *, page_size, kv_heads,
                            workspace=None, out=None):
     """Decode attention over the paged INT8 cache with the dequant fused in
@@ -217,19 +231,19 @@ def paged_decode_attention(q, k_pool, k_scales, v_pool, v_scales, page_table, le
         raise ValueError("q must be BF16 [batch, query_heads, 128]")
     for pool in (k_pool, v_pool):
         if pool.dtype != torch.int8 or pool.ndim < 3 or pool.shape[1] != page_size or \
-                pool[0, 0].numel() != kv_heads * head_dim:
+                _row_values(pool) != kv_heads * head_dim:
             raise ValueError("pools must be int8 [pages, page_size, kv_heads * 128]")
     for sc in (k_scales, v_scales):
         if sc.dtype != torch.float32 or sc.numel() != k_pool.shape[0] * page_size * kv_heads:
             raise ValueError("scales must be FP32 [pages, page_size, kv_heads]")
     batch, hq = q.shape[0], q.shape[1]
-    table = page_table.to(device=q.device, dtype=torch.int32).contiguous()
-    lens = lengths.to(device=q.device, dtype=torch.int32).contiguous()
+    table = _int32(page_table, q.device)
+    lens = _int32(lengths, q.device)
     if table.shape[0] != batch or lens.shape != (batch,):
         raise ValueError("page_table must be [batch, pages_per_seq] and lengths [batch]")
     pps = table.shape[1]
     lib = _lib.load()
-    need = int(lib.q6moe_attn_workspace_size(batch, hq, kv_heads, pps, page_size))
+    need = _attn_workspace_bytes(batch, hq, kv_heads, pps, page_size)
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     elif (not isinstance(workspace, torch.Tensor) or workspace.dtype != torch.uint8 or workspace.device != q.device
@@ -250,9 +264,7 @@ def paged_decode_attention(q, k_pool, k_scales, v_pool, v_scales, page_table, le
     a.pool_pages, a.pages_per_seq, a.page_size = k_pool.shape[0], pps, page_size
     a.out = out.data_ptr()
     a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
-    with torch.cuda.device(q.device):
-        rc = lib.q6moe_kv_decode_attention(ctypes.byref(a), _lib.stream_handle(q.device))
-    _lib.check(rc, "kv_decode_attention")
+    _launch.run("kv_decode_attention", lib.q6moe_kv_decode_attention, q.device, ctypes.byref(a))
     return out
 
 
@@ -269,11 +281,8 @@ def gather_scale_plane(plane, indices, groups, *, method="indexed"):
         raise ValueError("plane must be a GPU tensor")
     batch, sel = indices.shape
     plane = plane.contiguous()
-    idx = indices.to(device=plane.device, dtype=torch.int32).contiguous()
+    idx = _int32(indices, plane.device)
     out = torch.empty((batch, sel, groups), dtype=plane.dtype, device=plane.device)
-    lib = _lib.load()
-    with torch.cuda.device(plane.device):
-        rc = lib.q6moe_kv_gather_scales(plane.data_ptr(), _dtype_code(plane.dtype), idx.data_ptr(), batch, sel,
-                                        groups, plane.shape[1], out.data_ptr(), _lib.stream_handle(plane.device))
-    _lib.check(rc, "kv_gather_scales")
+    _launch.run("kv_gather_scales", _lib.load().q6moe_kv_gather_scales, plane.device, plane.data_ptr(),
+                _dtype_code(plane.dtype), idx.data_ptr(), batch, sel, groups, plane.shape[1], out.data_ptr())
     return out

@@ -12,7 +12,7 @@ multiplies with FP32 accumulation. ``pack_q8`` is the reference's packer.
 
 import torch
 
-from . import _lib
+from . import _launch, _lib
 from .experts import _CACHE, pack_experts
 from .quant import dequantize_rows
 from .quantize import quantize_q8_0 as pack_q8
@@ -45,10 +45,8 @@ def q8_matmul(x, packed, *, output_dtype=None):
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     lib = _lib.load()
     ws = torch.empty(int(lib.q6moe_q8_matmul_workspace_size(m, k)), dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = lib.q6moe_q8_matmul(x.data_ptr(), m, k, table.data.data_ptr(), n, y.data_ptr(), ws.data_ptr(),
-                                 ws.numel(), _lib.stream_handle(x.device))
-    _lib.check(rc, "q8_matmul")
+    _launch.run("q8_matmul", lib.q6moe_q8_matmul, x.device, x.data_ptr(), m, k, table.data.data_ptr(), n, y.data_ptr(),
+                ws.data_ptr(), ws.numel())
     return y
 
 

@@ -35,7 +35,7 @@ from functools import lru_cache
 import numpy as np
 import torch
 
-from . import _lib
+from . import _launch, _lib
 from .quant import BLOCK_LAYOUTS
 
 EXPERT_ROW_TILE = 128
@@ -63,13 +63,17 @@ class ExpertTable:
 
     def c_table(self):
         t = _lib.Table()
+        self.fill(t)
+        return t
+
+    def fill(self, t):
+        """Writes this table into the C structure ``t`` (zeroed, as ctypes makes it)."""
         t.qtype = _lib.QTYPE_CODES[self.qtype]
         t.data = self.data.data_ptr()
         t.data_stride = self.data.stride(0) if self.data.ndim > 1 else 0
         if self.scales is not None:
             t.scales = self.scales.data_ptr()
             t.scale_stride = self.scales.stride(0) if self.scales.ndim > 1 else 0
-        return t
 
     def nbytes(self):
         return self.data.numel() + (0 if self.scales is None else self.scales.numel())
@@ -191,7 +195,7 @@ def _as_table(t, qtype, rows, width, name):
     if isinstance(t, ExpertTable):
         if t.qtype != qtype or t.rows != rows or t.width != width:
             raise ValueError(f"{name} table holds {t.qtype} [{t.rows}, {t.width}], expected {qtype} [{rows}, {width}]")
-        if t.data.device.type != "cuda":
+        if not t.data.is_cuda:
             raise ValueError("expert tables must be on a GPU device")
         return t
     if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
@@ -234,6 +238,12 @@ def _check_workspace(workspace, need, device):
     return workspace
 
 
+@lru_cache(maxsize=256)
+def _workspace_bytes(tokens, top_k, experts, hidden, intermediate, shared_intermediate):
+    return int(_lib.load().q6moe_moe_workspace_size(tokens, top_k, experts, hidden, intermediate,
+                                                    shared_intermediate))
+
+
 MODES = (0, 1, 2)  # kernel family: by token count, decode-step kernels, grouped (prefill) kernels
 
 
@@ -267,8 +277,7 @@ class ExpertFFN:
         return ExpertFFN(self.qtype, self.hidden, self.intermediate, mode, self.down_qtype, self.compute)
 
     def workspace_bytes(self, tokens, top_k, experts, shared_intermediate=0):
-        return int(_lib.load().q6moe_moe_workspace_size(
-            tokens, top_k, experts, self.hidden, self.intermediate, shared_intermediate))
+        return _workspace_bytes(tokens, top_k, experts, self.hidden, self.intermediate, shared_intermediate)
 
     def prepare(self, gate, up, down, device=None):
         """Pack a layer's raw GGUF tables ([E, bytes_per_expert] uint8, host or
@@ -283,10 +292,7 @@ class ExpertFFN:
         """Routed FFN of x [B, hidden] BF16 through ``q6moe_moe_forward``; see ``args``."""
         args, out, keep = self.args(gate, up, down, x, ids, weights, shared=shared, workspace=workspace, out=out,
                                     events=events)
-        lib = _lib.load()
-        with torch.cuda.device(x.device):
-            rc = lib.q6moe_moe_forward(ctypes.byref(args), _lib.stream_handle(x.device))
-        _lib.check(rc, "moe_forward")
+        _launch.run("moe_forward", _lib.load().q6moe_moe_forward, x.device, ctypes.byref(args))
         del keep
         return out
 
@@ -315,7 +321,7 @@ class ExpertFFN:
         experts = gate.experts
         if up.experts != experts or down.experts != experts:
             raise ValueError("gate, up and down must hold the same number of experts")
-        if not isinstance(x, torch.Tensor) or x.device.type != "cuda":
+        if not isinstance(x, torch.Tensor) or not x.is_cuda:
             raise ValueError("x must be a GPU tensor")
         if x.dtype != torch.bfloat16 or x.ndim != 2 or x.shape[1] != H or x.shape[0] < 1:
             raise ValueError(f"x must be a nonempty BF16 [tokens, {H}] tensor")
@@ -325,10 +331,16 @@ class ExpertFFN:
             raise ValueError("routing weights must have x's dtype (BF16)")
         B, K = ids.shape
         x = x.contiguous()
-        ids = ids.to(device=x.device, dtype=torch.int32).contiguous()
-        weights = weights.to(x.device).contiguous()
+        device = x.device
+        if ids.dtype is not torch.int32 or ids.device != device:
+            ids = ids.to(device=device, dtype=torch.int32)
+        if weights.device != device:
+            weights = weights.to(device)
+        ids, weights = ids.contiguous(), weights.contiguous()
         args = _lib.MoeArgs()
-        args.gate, args.up, args.down = gate.c_table(), up.c_table(), down.c_table()
+        gate.fill(args.gate)
+        up.fill(args.up)
+        down.fill(args.down)
         args.experts, args.hidden, args.intermediate = experts, H, I
         args.x, args.ids, args.weights = x.data_ptr(), ids.data_ptr(), weights.data_ptr()
         args.tokens, args.top_k = B, K
@@ -339,7 +351,9 @@ class ExpertFFN:
             sg = _as_table(shared["gate"], q, Is, H, "shared gate")
             su = _as_table(shared["up"], q, Is, H, "shared up")
             sd = _as_table(shared["down"], qd, H, Is, "shared down")
-            args.shared_gate, args.shared_up, args.shared_down = sg.c_table(), su.c_table(), sd.c_table()
+            sg.fill(args.shared_gate)
+            su.fill(args.shared_up)
+            sd.fill(args.shared_down)
             args.shared_intermediate = Is
             scale, router = shared.get("scale"), shared.get("router")
             if scale is not None and router is not None:

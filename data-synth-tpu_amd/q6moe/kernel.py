@@ -12,7 +12,7 @@ call compatibility and ignored: there is no interpreter or CPU path.
 
 import torch
 
-from . import _lib
+from . import _launch, _lib
 from .layout import OUTPUT_TILE, QK, SCALE_FETCH_BYTES, SCALE_TILE_BYTES, TILE_BYTES
 
 
@@ -25,7 +25,7 @@ def _plane_sizes(output_features, inputs):
 
 def _require_device(*tensors):
     for t in tensors:
-        if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
             raise ValueError("q6moe operators take torch tensors on a GPU device")
 
 
@@ -55,14 +55,9 @@ def q6_matmul(x, packed, scales, *, output_features, batch_tile=8, interpret=Fal
     x = x if x.stride(1) == 1 else x.contiguous()
     packed, scales = packed.contiguous(), scales.contiguous()
     y = torch.empty((m, output_features), dtype=out_dtype, device=x.device)
-    lib = _lib.load()
-    with torch.cuda.device(x.device):
-        rc = lib.q6moe_q6_matmul(
-            _lib.ptr(x), m, inputs, x.stride(0), _lib.ptr(packed), _lib.ptr(scales),
-            output_features, _lib.ptr(y), _lib.BF16 if out_dtype == torch.bfloat16 else _lib.F32,
-            output_features, _lib.stream_handle(x.device),
-        )
-    _lib.check(rc, "q6_matmul")
+    _launch.run("q6_matmul", _lib.load().q6moe_q6_matmul, x.device, x.data_ptr(), m, inputs, x.stride(0),
+                packed.data_ptr(), scales.data_ptr(), output_features, y.data_ptr(),
+                _lib.BF16 if out_dtype == torch.bfloat16 else _lib.F32, output_features)
     return y
 
 

@@ -8,7 +8,7 @@ FP32 or BF16 (RNE of the FP32 value, as ``astype(bfloat16)`` does).
 
 import torch
 
-from . import _lib
+from . import _launch, _lib
 
 BLOCK_LAYOUTS = {
     "Q4_K": (256, 144),
@@ -92,11 +92,8 @@ def dequantize_rows(raw, qtype, row_width, dtype=None, backend="hip"):
     for s in lead:
         rows *= s
     out = torch.empty(lead + (row_width,), dtype=dtype, device=raw.device)
-    lib = _lib.load()
-    with torch.cuda.device(raw.device):
-        rc = lib.q6moe_gguf_decode(
-            _lib.ptr(raw.contiguous()), _lib.GGUF_TYPE_CODES[name], rows, row_width, _lib.ptr(out),
-            _lib.BF16 if dtype == torch.bfloat16 else _lib.F32, _lib.stream_handle(raw.device),
-        )
-    _lib.check(rc, "dequantize_rows")
+    raw = raw.contiguous()
+    _launch.run("dequantize_rows", _lib.load().q6moe_gguf_decode, raw.device, raw.data_ptr(),
+                _lib.GGUF_TYPE_CODES[name], rows, row_width, out.data_ptr(),
+                _lib.BF16 if dtype == torch.bfloat16 else _lib.F32)
     return out

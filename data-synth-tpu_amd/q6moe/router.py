@@ -9,11 +9,11 @@ weights divided by their sum, inactive rows zeroed, RNE to BF16.
 
 import torch
 
-from . import _lib
+from . import _launch, _lib
 
 
 def routes(logits, top_k, active=None):
-    if not isinstance(logits, torch.Tensor) or logits.device.type != "cuda" or logits.ndim != 2:
+    if not isinstance(logits, torch.Tensor) or not logits.is_cuda or logits.ndim != 2:
         raise ValueError("logits must be a GPU tensor [tokens, experts]")
     logits = logits.to(torch.float32).contiguous()
     B, E = logits.shape
@@ -26,9 +26,6 @@ def routes(logits, top_k, active=None):
             raise ValueError("active must hold one flag per token")
     ids = torch.empty((B, top_k), dtype=torch.int32, device=logits.device)
     weights = torch.empty((B, top_k), dtype=torch.bfloat16, device=logits.device)
-    lib = _lib.load()
-    with torch.cuda.device(logits.device):
-        rc = lib.q6moe_route_topk(logits.data_ptr(), B, E, top_k, None if act is None else act.data_ptr(),
-                                  ids.data_ptr(), weights.data_ptr(), _lib.stream_handle(logits.device))
-    _lib.check(rc, "route_topk")
+    _launch.run("route_topk", _lib.load().q6moe_route_topk, logits.device, logits.data_ptr(), B, E, top_k,
+                None if act is None else act.data_ptr(), ids.data_ptr(), weights.data_ptr())
     return ids, weights
