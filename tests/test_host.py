@@ -173,3 +173,15 @@ def test_expert_ffn_mode_copies_leave_the_cached_callable_alone():
         fn.mode = 1
     with pytest.raises(ValueError):
         fn.with_mode(3)
+
+
+def test_launch_refuses_tensors_off_the_gpu():
+    import torch
+    from q6moe import _launch
+
+    def called(*args):
+        raise AssertionError("reached the library")
+
+    for device in (torch.device("cpu"), torch.device("cpu", 0)):
+        with pytest.raises(ValueError, match="Expected a cuda device"):
+            _launch.run("x", called, device, 1)
