@@ -18,7 +18,7 @@
 //      heads as B operand; scores go to the workspace as BF16, and each
 //      wave's maximum m_w and sum l_w of exp(score - m_w) over its 64 tokens.
 //   2. attn_pv_kernel: per 2048-token chunk (8 waves, four 64-token tiles
-//      each), wave h first merges head h's statistics over the attended
+//      each; 1024 or 512 tokens for few sequences), wave h first merges head h's statistics over the attended
 //      tokens, max = max_w m_w and sum = sum_w l_w exp(m_w - max) in a fixed
 //      order; the workgroup forms RNE_bf16(prob) once per (head, token) in
 //      LDS; each wave then runs P.V for its tiles, in turn, on MFMA with the
@@ -40,8 +40,7 @@ constexpr int kAttnChunk = 256;  // tokens per scores workgroup: 4 waves x 64
 constexpr int kAttnWaveTok = 64;
 constexpr int kPvWaves = 8;      // waves per P.V workgroup
 constexpr int kPvThreads = kPvWaves * 64;
-constexpr int kPvTiles = 4;      // 64-token tiles per P.V wave
-constexpr int kPvChunk = kPvTiles * kPvThreads;  // tokens per P.V workgroup (one partial sum)
+constexpr int kPvMaxTiles = 4;   // most 64-token tiles per P.V wave; tiles x kPvThreads tokens per workgroup
 
 struct AttnParams {
   const uint16_t* q;                 // [B, Hq, D]
@@ -52,7 +51,8 @@ struct AttnParams {
   const int32_t* table;              // [B, pps]
   const int32_t* len;                // [B]
   int64_t pool_pages;
-  int pps, page, kvh, hq, r, cap, nchunks;  // nchunks: P.V chunks of kPvChunk tokens
+  int pps, page, kvh, hq, r, cap, nchunks;  // nchunks: P.V chunks of pv_tiles * kPvThreads tokens
+  int pv_tiles;
   uint16_t* s;                       // [B, Hq, cap] BF16 scores
   float* wstats;                     // [B, Hq, cap / 64, 2]: per 64 tokens, max m_w and sum of exp(score - m_w)
   float* part;                       // [B, KVH, nchunks, kAttnR, D]
@@ -98,7 +98,11 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnParams p) {
       qb[ks] = live ? v : u32x4{0u, 0u, 0u, 0u};
     }
   }
-  const float kDiv = static_cast<float>(11.313708498984761);  // float32(128 ** 0.5) (attention_cache.py:163)
+  // RNE_bf16(raw / float32(128 ** 0.5)) (attention_cache.py:163) as a product
+  // with the rounded reciprocal: the BF16 result is the same for every one of
+  // the 65536 BF16 values of raw (a test checks them), and the quotient took ten
+  // instructions of each score.
+  const float kInv = 1.f / static_cast<float>(11.313708498984761);
   const int64_t rowbytes = (int64_t)p.kvh * kAttnD;
   const int64_t base = attn_row(p, attn_page(p, b, t0), t0);
   // the wave's rows start at pool row base (wave-uniform); the lane adds its
@@ -144,7 +148,7 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnParams p) {
     // lane holds tokens t0 + 16rb + 4g + [0, 4) of query head col
     const int tt = t0 + 16 * rb + 4 * g;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) sv[rb][v] = bf16_round(bf16_round(acc[v]) / kDiv);
+    for (int v = 0; v < 4; ++v) sv[rb][v] = bf16_round(bf16_round(acc[v]) * kInv);
     if (col < p.r) {
       uint16_t* dst = p.s + ((int64_t)b * p.hq + kh * p.r + col) * p.cap + tt;
       *reinterpret_cast<u32x2*>(dst) = u32x2{pack_bf16x2(sv[rb][0], sv[rb][1]), pack_bf16x2(sv[rb][2], sv[rb][3])};
@@ -176,7 +180,9 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnParams p) {
   }
 }
 
+template <int kPvTiles>
 __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu(4))) attn_pv_kernel(AttnParams p) {
+  constexpr int kPvChunk = kPvTiles * kPvThreads;  // tokens per workgroup (one partial sum)
   __shared__ __attribute__((aligned(16))) uint16_t pr[kAttnR][kPvChunk];  // RNE_bf16(prob) [head][token]
   __shared__ float red[kPvWaves][kAttnR][kAttnD];                       // per-wave partial sums
   const int chunk = blockIdx.x, kh = blockIdx.y, b = blockIdx.z;
@@ -211,7 +217,7 @@ __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu
   // order (the first 8 in one batch of loads), max over them and a fixed xor
   // tree, then sum of l_w exp(m_w - max) the same way; every workgroup of the
   // head computes the same values.
-  float sm[kAttnR], sl[kAttnR];
+  float sm[kAttnR], sl[kAttnR], si[kAttnR];  // the heads' maximum, sum and the sum's rounded reciprocal
   {
     const int nw = (n + kAttnWaveTok - 1) / kAttnWaveTok;
     const f32x2* wsh = reinterpret_cast<const f32x2*>(p.wstats) +
@@ -248,6 +254,7 @@ __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu
       const f32x2 v = s_st[h < p.r ? h : 0];
       sm[h] = v[0];
       sl[h] = v[1];
+      si[h] = 1.f / v[1];
     }
   }
   // V codes of a tile: lane (r16, kg) reads channels 8*r16 + [0, 8) of the
@@ -291,7 +298,15 @@ __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu
     for (int h = 0; h < kAttnR; ++h) {
       const int tt = t + kPvThreads * i;
       float q = 0.f;
-      if (tt < nv && h < p.r) q = bf16_round(expf(bf16_to_float(sc[i][h]) - sm[h]) / sl[h]);
+      if (tt < nv && h < p.r) {
+        // exp(score - max) / sum, the correctly rounded quotient (Markstein, IBM
+        // J. Res. Dev. 34, 1990): the rounded reciprocal's product and one
+        // correction by the exact FMA residual, three instructions for each of
+        // the head's tokens
+        const float e = expf(bf16_to_float(sc[i][h]) - sm[h]);
+        q = e * si[h];
+        q = bf16_round(__builtin_fmaf(__builtin_fmaf(-q, sl[h], e), si[h], q));
+      }
       pr[h][tt] = bf16_bits(q);
     }
   mask_tile(0);
@@ -352,7 +367,8 @@ __global__ void __launch_bounds__(8 * kAttnD) attn_combine_kernel(AttnParams p) 
   __shared__ float red[8][kAttnD];
   const int h = blockIdx.x, b = blockIdx.y, d = threadIdx.x % kAttnD, grp = threadIdx.x / kAttnD;
   const int kh = h / p.r, hr = h % p.r;
-  const int nc = (attn_len(p, b) + kPvChunk - 1) / kPvChunk;
+  const int pv_chunk = p.pv_tiles * kPvThreads;
+  const int nc = (attn_len(p, b) + pv_chunk - 1) / pv_chunk;
   const int per = (nc + 7) / 8, cb = grp * per, ce = cb + per < nc ? cb + per : nc;
   const float* src = p.part + (((int64_t)b * p.kvh + kh) * p.nchunks) * kAttnR * kAttnD + hr * kAttnD + d;
   float v = 0.f;
@@ -381,9 +397,19 @@ struct AttnLayout {
 
 static size_t attn_align(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// 64-token tiles per P.V wave: four (2048 tokens per workgroup) where that gives
+// every CU a workgroup, fewer for few sequences, KV heads or pages. One sequence
+// of 32 K tokens over 4 KV heads: 17.8 us with 64 workgroups of 2048 tokens, 9.8
+// us with 256 of 512; 4 K tokens 17.2 and 9.0 us.
+static int attn_pv_tiles(int64_t B, int64_t kvh, int64_t cap) {
+  int tiles = kPvMaxTiles;
+  while (tiles > 1 && B * kvh * cdiv(cap, tiles * kPvThreads) < 256) tiles /= 2;
+  return tiles;
+}
+
 static AttnLayout attn_layout(int64_t B, int64_t hq, int64_t kvh, int64_t cap) {
   AttnLayout L;
-  const int64_t nchunks = (cap + kPvChunk - 1) / kPvChunk;
+  const int64_t nchunks = cdiv(cap, attn_pv_tiles(B, kvh, cap) * kPvThreads);
   L.s = 0;
   L.wstats = attn_align(L.s + (size_t)B * hq * cap * 2);
   L.part = attn_align(L.wstats + (size_t)B * hq * (cap / kAttnWaveTok) * 2 * 4);
@@ -439,7 +465,8 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   p.hq = (int)a->query_heads;
   p.r = (int)(a->query_heads / a->kv_heads);
   p.cap = (int)cap;
-  p.nchunks = (int)((cap + kPvChunk - 1) / kPvChunk);
+  p.pv_tiles = attn_pv_tiles(a->batch, p.kvh, cap);
+  p.nchunks = (int)cdiv(cap, p.pv_tiles * kPvThreads);
   uint8_t* w = reinterpret_cast<uint8_t*>(a->workspace);
   p.s = reinterpret_cast<uint16_t*>(w + L.s);
   p.wstats = reinterpret_cast<float*>(w + L.wstats);
@@ -449,7 +476,12 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   const dim3 chunks((unsigned)((cap + kAttnChunk - 1) / kAttnChunk), (unsigned)p.kvh, (unsigned)a->batch);
   const dim3 pv_chunks((unsigned)p.nchunks, (unsigned)p.kvh, (unsigned)a->batch);
   hipLaunchKernelGGL(attn_scores_kernel, chunks, dim3(256), 0, s, p);
-  hipLaunchKernelGGL(attn_pv_kernel, pv_chunks, dim3(kPvThreads), 0, s, p);
+  if (p.pv_tiles == 4)
+    hipLaunchKernelGGL(attn_pv_kernel<4>, pv_chunks, dim3(kPvThreads), 0, s, p);
+  else if (p.pv_tiles == 2)
+    hipLaunchKernelGGL(attn_pv_kernel<2>, pv_chunks, dim3(kPvThreads), 0, s, p);
+  else
+    hipLaunchKernelGGL(attn_pv_kernel<1>, pv_chunks, dim3(kPvThreads), 0, s, p);
   hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)p.hq, (unsigned)a->batch), dim3(8 * kAttnD), 0, s, p);
   return check_launch("decode_attention kernels");
 }

@@ -129,3 +129,20 @@ def test_decode_attention_seeded_sweep(device, seed):
     sz = [np.concatenate([s, np.zeros((1,) + s.shape[1:], s.dtype)]) for s in scales]
     tz = np.where((table < 0) | (table >= pages), pages, table).astype(np.int32)
     _check(got, _want(pz, sz, tz, qv, lengths, page_size, kvh))
+
+
+@pytest.mark.parametrize("batch,kvh,pps,lengths", [
+    (1, 2, 20, [[511], [512], [513], [1024], [1025], [1280]]),            # 512-token chunks
+    (16, 8, 32, [[1023, 1024, 1025, 2048, 1, 64, 65, 1536] * 2]),         # 1024-token chunks
+    (16, 8, 40, [[2047, 2048, 2049, 2560, 1, 1537, 65, 511] * 2]),        # 2048-token chunks
+])
+def test_decode_attention_chunk_widths(device, batch, kvh, pps, lengths):
+    # The P.V workgroups take 512, 1024 or 2048 tokens by the call's size; the
+    # sequences share physical pages, so a small pool holds them. Every sequence
+    # up to 8 and the last one are checked.
+    pages, page_size, r = 48, 64, 4
+    pools, scales, table, q = _case(77 + batch, batch, kvh, r, pages=pages, page_size=page_size, pps=pps)
+    rows = sorted({*range(min(batch, 8)), batch - 1})
+    for lens in lengths:
+        got, qv = _run(device, pools, scales, table, q, lens, page_size, kvh)
+        _check(got[rows], _want(pools, scales, table, qv, lens, page_size, kvh, rows=rows))

@@ -185,3 +185,17 @@ def test_launch_refuses_tensors_off_the_gpu():
     for device in (torch.device("cpu"), torch.device("cpu", 0)):
         with pytest.raises(ValueError, match="Expected a cuda device"):
             _launch.run("x", called, device, 1)
+
+
+def test_score_scaling_by_the_reciprocal_is_exact_in_bf16():
+    # RNE_bf16(x / d) == RNE_bf16(x * RN(1 / d)) for d = float32(128 ** 0.5) and
+    # every BF16 x (the attention kernel multiplies)
+    x = (np.arange(65536, dtype=np.uint32) << 16).view(np.float32)
+    x = x[~np.isnan(x)]
+    d = np.float32(128 ** 0.5)
+
+    def bf16(v):
+        u = v.view(np.uint32).astype(np.uint64)
+        return (u + 0x7FFF + ((u >> 16) & 1)) >> 16
+
+    np.testing.assert_array_equal(bf16(x / d), bf16(x * (np.float32(1) / d)))
