@@ -850,7 +850,8 @@ static WsLayout ws_layout(int64_t B, int64_t K, int64_t E, int64_t H, int64_t I,
   return L;
 }
 
-constexpr int64_t kPrefillTile = 128;  // routes per prefill tile (moe_prefill.hip kM)
+constexpr int64_t kPrefillTile = 128;  // most routes per prefill tile (moe_tile.h kM)
+constexpr int64_t kThinTile = 64;      // and where experts see few routes
 
 static Proj make_proj(const q6moe_table& t, int rows, int k) {
   Proj p;
@@ -1488,7 +1489,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   const TokenSrc dense{1, (int)B, nullptr, nullptr, nullptr, nullptr};
   const auto shared_gate_up = [&] {  // in a launch of its own
     if (sh_tiled_gu)
-      launch_moe_prefill_gate_up(fmt, sg, su, ws, 0, a->x, (int)B, (int)H, (int)Is,
+      launch_moe_prefill_gate_up(fmt, sg, su, ws, (int)kPrefillTile, 0, a->x, (int)B, (int)H, (int)Is,
                                  pf_dense_gate_up(sg, su, a->x, (int)B, ws.sh_act), s, nullptr, nullptr);
     else
       dispatch_format(fmt, [&](auto fg) {
@@ -1497,7 +1498,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   };
   const auto shared_down = [&] {
     if (sh_tiled_dn)
-      launch_moe_prefill_down(fmt_dn, sd, ws, 0, (int)B, (int)H, (int)Is,
+      launch_moe_prefill_down(fmt_dn, sd, ws, (int)kPrefillTile, 0, (int)B, (int)H, (int)Is,
                               pf_dense_down(sd, ws.sh_act, (int)B, ws.sh_y), s);
     else
       dispatch_format(fmt_dn, [&](auto fd) {
@@ -1555,6 +1556,27 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     mark(4);
     return rc;
   }
+  // int8_q8 policy: the Q8_0 projections run W8A8 (compute.py:20-34)
+  const bool w8_gu = w8 && fmt == FMT_Q8, w8_dn = w8 && fmt_dn == FMT_Q8;
+  // The tiled MFMA kernels address token rows with 32-bit byte offsets.
+  const bool rows32 = B * H * 2 < (1ll << 31) && B * K * I * 2 < (1ll << 31);
+  const bool tiled_gu = !w8_gu && rows32 && pf_gate_up_supported(fmt, H, I);
+  const bool tiled_dn = !w8_dn && rows32 && pf_down_supported(fmt_dn, H, I);
+  // the shared expert's items in the routed launches
+  const bool join_gu = sh_tiled_gu && tiled_gu, join_dn = sh_tiled_dn && tiled_dn;
+  // Tiles of 64 routes up to 48 routes per expert on average: three waves per
+  // SIMD decode faster than the second 64 routes of a tile save. 512-expert
+  // top-10 Q6_K/Q8_0 layer, step: 200 tokens 475 us with 128 and 457 with 64,
+  // 2001 tokens 621 and 585; 128-expert top-8 layer: 128 tokens 132 and 124 us,
+  // 512 tokens 157 and 150, 768 (48 per expert) 168 and 168, 1024 183 and 195. Same
+  // outputs. Their more tile records take the place of the W8A8 policy's
+  // buffers, unused here, where these are large enough.
+  const int64_t thin_bytes = (int64_t)sizeof(PfTile) * (E + B * K / kThinTile + 1);
+  const bool thin = B * K <= 48 * E && !w8 && !join_gu && !join_dn && (tiled_gu || tiled_dn) &&
+                    thin_bytes <= (int64_t)(L.total - L.xq);
+  const int mtile = (int)(thin ? kThinTile : kPrefillTile);
+  const int max_tiles = (int)(E + B * K / mtile + 1);
+  if (thin) ws.tile = reinterpret_cast<PfTile*>(w + L.xq);
   mark(0);
   {
     static std::atomic<uint64_t> attr_done{0};
@@ -1578,7 +1600,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
       const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);
       const dim3 grid(1 + (unsigned)cdiv(gate.tokens, lanes / 64));
       hipLaunchKernelGGL(moe_route_small_kernel, grid, dim3(lanes), scatter_lds(K, E) + (size_t)E * 4, s, a->ids,
-                         a->weights, (int)B, (int)K, (int)E, (int)kPrefillTile, ws, gate);
+                         a->weights, (int)B, (int)K, (int)E, mtile, ws, gate);
     } else {
       const dim3 grid((unsigned)(nchunks + cdiv(gate.tokens, kChunk / 64)));
       hipLaunchKernelGGL(moe_route_count_kernel, grid, dim3(kChunk), (size_t)kChunk * K * 8, s, a->ids, a->weights,
@@ -1587,10 +1609,10 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
         // the scan folded into the scatter workgroups (up to 8192 tokens)
         const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);
         hipLaunchKernelGGL(moe_route_scan_scatter_kernel, dim3(nchunks), dim3(lanes), scatter_lds(K, E), s, a->ids,
-                           (int)B, (int)K, (int)E, nchunks, (int)kPrefillTile, ws, chunk_cnt);
+                           (int)B, (int)K, (int)E, nchunks, mtile, ws, chunk_cnt);
       } else {
         hipLaunchKernelGGL(moe_route_scan_kernel, dim3(1), dim3((unsigned)cdiv(E, 64) * 64), 0, s, (int)E, nchunks,
-                           (int)kPrefillTile, ws, chunk_cnt);
+                           mtile, ws, chunk_cnt);
         hipLaunchKernelGGL(moe_route_scatter_kernel, dim3(nchunks), dim3(kChunk), scatter_lds(K, E), s, a->ids,
                            (int)B, (int)K, (int)E, nchunks, ws, chunk_cnt);
       }
@@ -1603,19 +1625,6 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   const Proj g = make_proj(a->gate, (int)I, (int)H), u = make_proj(a->up, (int)I, (int)H),
              d = make_proj(a->down, (int)H, (int)I);
   const int max_tokens = (int)B;  // an expert sees each token at most once
-  // int8_q8 policy: the Q8_0 projections run W8A8 (compute.py:20-34)
-  const bool w8_gu = w8 && fmt == FMT_Q8, w8_dn = w8 && fmt_dn == FMT_Q8;
-  // The tiled MFMA kernels address token rows with 32-bit byte offsets.
-  const bool rows32 = B * H * 2 < (1ll << 31) && B * K * I * 2 < (1ll << 31);
-  const bool tiled_gu = !w8_gu && rows32 && pf_gate_up_supported(fmt, H, I);
-  const bool tiled_dn = !w8_dn && rows32 && pf_down_supported(fmt_dn, H, I);
-  const int max_tiles = (int)(E + B * K / kPrefillTile + 1);
-  if ((tiled_gu || tiled_dn) && pf_tile_routes() != kPrefillTile) {
-    set_error("moe_forward: prefill tile size mismatch");
-    return Q6MOE_ERR_HIP;
-  }
-  // the shared expert's items in the routed launches
-  const bool join_gu = sh_tiled_gu && tiled_gu, join_dn = sh_tiled_dn && tiled_dn;
   if (Is && !join_gu) shared_gate_up();
   // W8A8: tiled unless the items (active experts x column blocks) would leave
   // the chip idle and no expert has more than a 64-token tile; there the kernel
@@ -1638,7 +1647,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   } else if (tiled_gu) {
     // events[1] and [2] take the gate/up kernel's own start and end timestamps
     const PfDense D = join_gu ? pf_dense_gate_up(sg, su, a->x, (int)B, ws.sh_act) : PfDense{};
-    launch_moe_prefill_gate_up(fmt, g, u, ws, max_tiles, a->x, (int)B, (int)H, (int)I, D, s,
+    launch_moe_prefill_gate_up(fmt, g, u, ws, mtile, max_tiles, a->x, (int)B, (int)H, (int)I, D, s,
                                a->events ? a->events[1] : nullptr, a->events ? a->events[2] : nullptr);
   } else {
     mark(1);
@@ -1659,7 +1668,7 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
       launch_w8(false, d, d, routed, slots, 1, src, ws.y, s);
   } else if (tiled_dn) {
     const PfDense D = join_dn ? pf_dense_down(sd, ws.sh_act, (int)B, ws.sh_y) : PfDense{};
-    launch_moe_prefill_down(fmt_dn, d, ws, max_tiles, (int)(B * K), (int)H, (int)I, D, s);
+    launch_moe_prefill_down(fmt_dn, d, ws, mtile, max_tiles, (int)(B * K), (int)H, (int)I, D, s);
   } else {
     dispatch_format(fmt_dn, [&](auto fd) {
       launch_down<decltype(fd)::value>(d, routed, slots, max_tokens, ws.act, (int)H, (int)I, ws.y, s);

@@ -237,10 +237,10 @@ int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStre
 // intermediate a multiple of 128, hidden of 128), each launched on its own.
 bool pf_gate_up_supported(int fmt, int64_t H, int64_t I);
 bool pf_down_supported(int fmt, int64_t H, int64_t I);
-int64_t pf_tile_routes();
 // A dense expert (the always-on shared one: every token, weight 1) whose items
 // run in the tiled launches with the routed ones; tiles == 0: none. max_tiles
-// == 0 in the launches below: no routed items (``ws`` is then not read).
+// == 0 in the launches below: no routed items (``ws`` is then not read); mtile:
+// most routes per routed tile, 64 or 128 (128 with dense items).
 struct PfDense {
   Proj p0, p1;         // gate and up, or down (p0)
   const uint16_t* in;  // x [tokens, H], or the activations [tokens, p0.k]
@@ -250,10 +250,10 @@ struct PfDense {
 };
 PfDense pf_dense_gate_up(const Proj& g, const Proj& u, const uint16_t* x, int tokens, uint16_t* act);
 PfDense pf_dense_down(const Proj& d, const uint16_t* act, int tokens, uint16_t* y);
-int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles,
+int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int mtile, int max_tiles,
                                const uint16_t* x, int B, int H, int I, const PfDense& D, hipStream_t s,
                                void* gate_up_start, void* after_gate_up);
-int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I,
+int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int mtile, int max_tiles, int routes, int H, int I,
                             const PfDense& D, hipStream_t s);
 
 // W8A8 policy: quantised activations, codes [rows, k] and scales [rows, k / 32].

@@ -34,13 +34,20 @@ namespace q6moe {
 
 namespace pf {
 
-constexpr int kHalfBytes = kM * 128 * 2;  // one K half of the token tile (32 KB)
+// The kernels come for tiles of up to MT = 128 or 64 routes. 64: half the
+// accumulators and token rows, so that with Q6_K and Q8_0 weights three
+// workgroups share a CU (three waves per SIMD within 168 registers; the other
+// formats would spill) where the experts see few routes each and the weight
+// decode bounds the step.
+template <int MT>
+constexpr int kHalfBytes = MT * 128 * 2;  // one K half of the token tile (32 or 16 KB)
 constexpr int kXStages = 2;        // token-tile stages in LDS: the K half being multiplied and the next
 // A tile of NCG (2, 4, 6 or 8) 16-route column groups: the token rows of a K
 // half take NCG KB per wave, i.e. NCG DMA instructions of 1 KB per wave.
-constexpr int kLds = kXStages * kHalfBytes;
-
-static_assert(kLds <= 160 * 1024, "LDS budget");
+template <int MT>
+constexpr int kLds = kXStages * kHalfBytes<MT>;
+template <int FMT, int MT>
+constexpr int kWgPerCu = MT == 64 && (FMT == FMT_Q6 || FMT == FMT_Q8) ? 3 : 2;
 
 // The weights of one unit (a whole K block) in the registers of the lane that
 // decodes them (row j = lane % 16, k-group jA = lane / 16); both K halves
@@ -320,7 +327,7 @@ __device__ __forceinline__ void x_offsets(uint32_t (&xoff)[NCG], const int (&row
 // instructions at once right after the barrier.
 // kEven: K is a multiple of 256 (whole K blocks); the loop then runs its
 // steps in pairs with no branch between a block's two halves.
-template <int FMT, int NCG, bool kEven, typename RowFn, typename RowOf>
+template <int FMT, int MT, int NCG, bool kEven, typename RowFn, typename RowOf>
 __device__ __forceinline__ void pf_stream(uint8_t* smem, const Proj* projs, const int* unit_proj, RowFn rg_of,
                                           const uint16_t* x, int x_rows, RowOf row_of, int K, int64_t expert,
                                           f32x4 (&acc)[kUnits][NCG]) {
@@ -359,7 +366,7 @@ __device__ __forceinline__ void pf_stream(uint8_t* smem, const Proj* projs, cons
     if constexpr (part < 2) {
       static_assert(NCG % 2 == 0, "the token DMA splits evenly over two parts");
       constexpr int per = NCG / 2, i0 = part * per;
-      uint8_t* xs = smem + slot * kHalfBytes + wave * NCG * 1024;
+      uint8_t* xs = smem + slot * kHalfBytes<MT> + wave * NCG * 1024;
 #pragma unroll
       for (int i = i0; i < i0 + per; ++i) bdma16(xr, xoff[i], (uint32_t)(kb * kQK + h * 128) * 2u, xs + i * 1024);
     } else if constexpr (slot == 1 && part - 2 < kUnits) {
@@ -387,7 +394,7 @@ __device__ __forceinline__ void pf_stream(uint8_t* smem, const Proj* projs, cons
       if constexpr (slot == 0) wr[set][u].fold(lane);
     }
     const bool more = s + 1 < S;
-    const uint8_t* xs = smem + slot * kHalfBytes;
+    const uint8_t* xs = smem + slot * kHalfBytes<MT>;
     u32x4 a[kUnits][4];
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) wr[set][u].half(slot, lane, a[u]);  // slot == s % 2 == h
@@ -439,20 +446,27 @@ __device__ __forceinline__ void pf_stream(uint8_t* smem, const Proj* projs, cons
 // Calls f(std::integral_constant<int, NCG>) for the tile's column groups: its
 // valid routes rounded up to 32 (2, 4, 6 or 8 groups of 16), so a partial tile
 // issues only the MFMAs and token DMA of the routes it holds.
-template <typename F>
+template <int MT, typename F>
 __device__ __forceinline__ void with_column_groups(int nv, F&& f) {
-  switch ((nv + 31) >> 5) {
-    case 1: f(std::integral_constant<int, 2>{}); break;
-    case 2: f(std::integral_constant<int, 4>{}); break;
-    case 3: f(std::integral_constant<int, 6>{}); break;
-    default: f(std::integral_constant<int, 8>{}); break;
+  if constexpr (MT == 64) {
+    if (nv <= 32)
+      f(std::integral_constant<int, 2>{});
+    else
+      f(std::integral_constant<int, 4>{});
+  } else {
+    switch ((nv + 31) >> 5) {
+      case 1: f(std::integral_constant<int, 2>{}); break;
+      case 2: f(std::integral_constant<int, 4>{}); break;
+      case 3: f(std::integral_constant<int, 6>{}); break;
+      default: f(std::integral_constant<int, 8>{}); break;
+    }
   }
 }
 
 }  // namespace pf
 
-template <int FMT, bool kDense>
-__global__ void __launch_bounds__(64 * pf::kWaves, 2)
+template <int FMT, bool kDense, int MT>
+__global__ void __launch_bounds__(64 * pf::kWaves, (pf::kWgPerCu<FMT, MT>))
     moe_pf_gate_up_kernel(Proj gate, Proj up, MoeWs ws, const uint16_t* __restrict__ x, int tokens, int hidden,
                           uint16_t* __restrict__ act_r, int inter_r, int ncol, PfDense D) {
   using namespace pf;
@@ -467,7 +481,7 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
   const int wave = wave_id(), lane = threadIdx.x & 63;
   const int jA = lane >> 4, j = lane & 15;
   const int rgb = col * kWaves + wave;  // this wave's row group (gate and up)
-  with_column_groups(T.nv, [&](auto ncg_c) {
+  with_column_groups<MT>(T.nv, [&](auto ncg_c) {
     constexpr int NCG = decltype(ncg_c)::value;
     const Proj projs[2] = {dense ? D.p0 : gate, dense ? D.p1 : up};
     const int unit_proj[kUnits] = {0, 1};
@@ -481,10 +495,10 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
       return dense ? r : ws.route_tok[r];
     };
     if (hidden % 256 == 0)
-      pf_stream<FMT, NCG, true>(smem, projs, unit_proj, [&](int) { return rgb; }, x, tokens, row_of, hidden,
+      pf_stream<FMT, MT, NCG, true>(smem, projs, unit_proj, [&](int) { return rgb; }, x, tokens, row_of, hidden,
                                 T.expert, acc);
     else
-      pf_stream<FMT, NCG, false>(smem, projs, unit_proj, [&](int) { return rgb; }, x, tokens, row_of, hidden,
+      pf_stream<FMT, MT, NCG, false>(smem, projs, unit_proj, [&](int) { return rgb; }, x, tokens, row_of, hidden,
                                  T.expert, acc);
     const int row = rgb * 16 + 4 * jA;
 #pragma unroll
@@ -507,8 +521,8 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
   });
 }
 
-template <int FMT, bool kDense>
-__global__ void __launch_bounds__(64 * pf::kWaves, 2)
+template <int FMT, bool kDense, int MT>
+__global__ void __launch_bounds__(64 * pf::kWaves, (pf::kWgPerCu<FMT, MT>))
     moe_pf_down_kernel(Proj down, MoeWs ws, const uint16_t* __restrict__ act_r, int routes, int inter_r,
                        uint16_t* __restrict__ y_r, int hidden, int ncol, PfDense D) {
   using namespace pf;
@@ -524,7 +538,7 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
   const int wave = wave_id(), lane = threadIdx.x & 63;
   const int jA = lane >> 4, j = lane & 15;
   const int rgb = col * 2 * kWaves + 2 * wave;  // this wave's two row groups
-  with_column_groups(T.nv, [&](auto ncg_c) {
+  with_column_groups<MT>(T.nv, [&](auto ncg_c) {
     constexpr int NCG = decltype(ncg_c)::value;
     const Proj projs[1] = {dense ? D.p0 : down};
     const int unit_proj[kUnits] = {0, 0};
@@ -535,10 +549,10 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 2)
       for (int t = 0; t < NCG; ++t) acc[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto row_of = [&](int t) { return T.r0 + (t < T.nv ? t : T.nv - 1); };
     if (inter % 256 == 0)
-      pf_stream<FMT, NCG, true>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
+      pf_stream<FMT, MT, NCG, true>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
                                 T.expert, acc);
     else
-      pf_stream<FMT, NCG, false>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
+      pf_stream<FMT, MT, NCG, false>(smem, projs, unit_proj, [&](int u) { return rgb + u; }, act, act_rows, row_of, inter,
                                  T.expert, acc);
 #pragma unroll
     for (int u = 0; u < kUnits; ++u) {
@@ -567,7 +581,6 @@ bool pf_down_supported(int fmt, int64_t H, int64_t I) {
   return I % 128 == 0 && H % (32 * pf::kWaves) == 0;
 }
 
-int64_t pf_tile_routes() { return pf::kM; }
 
 template <typename F>
 static void dispatch_pf_format(int fmt, F&& f) {
@@ -595,61 +608,65 @@ PfDense pf_dense_down(const Proj& d, const uint16_t* act, int tokens, uint16_t* 
   return PfDense{d, d, act, y, tokens, pf_tiles(tokens), d.rows / (32 * pf::kWaves), d.rows};
 }
 
-template <int FMT, bool kDense>
+template <int FMT, bool kDense, int MT>
 static void pf_launch_gate_up(const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles, const uint16_t* x, int B,
                               int H, int I, const PfDense& D, hipStream_t s, void* gate_up_start, void* after_gate_up) {
   static std::atomic<uint64_t> attr_done{0};
   once_per_device(attr_done, [] {
-    (void)hipFuncSetAttribute((const void*)moe_pf_gate_up_kernel<FMT, kDense>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds);
+    (void)hipFuncSetAttribute((const void*)moe_pf_gate_up_kernel<FMT, kDense, MT>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds<MT>);
   });
   const int ncol = max_tiles ? I / (16 * pf::kWaves) : 0;
   const dim3 grid = pf_grid(ncol, max_tiles, D), block(64 * pf::kWaves);
   if (gate_up_start && after_gate_up) {
     // the events take the kernel's own start and end timestamps
-    hipExtLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense>), grid, block, pf::kLds, s, (hipEvent_t)gate_up_start,
+    hipExtLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense, MT>), grid, block, pf::kLds<MT>, s, (hipEvent_t)gate_up_start,
                           (hipEvent_t)after_gate_up, 0, g, u, ws, x, B, H, ws.act, I, ncol, D);
   } else {
-    hipLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense>), grid, block, pf::kLds, s, g, u, ws, x, B, H, ws.act, I,
+    hipLaunchKernelGGL((moe_pf_gate_up_kernel<FMT, kDense, MT>), grid, block, pf::kLds<MT>, s, g, u, ws, x, B, H, ws.act, I,
                        ncol, D);
     if (after_gate_up) (void)hipEventRecord((hipEvent_t)after_gate_up, s);
   }
 }
 
-template <int FMT, bool kDense>
+template <int FMT, bool kDense, int MT>
 static void pf_launch_down(const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I, const PfDense& D,
                            hipStream_t s) {
   static std::atomic<uint64_t> attr_done{0};
   once_per_device(attr_done, [] {
-    (void)hipFuncSetAttribute((const void*)moe_pf_down_kernel<FMT, kDense>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds);
+    (void)hipFuncSetAttribute((const void*)moe_pf_down_kernel<FMT, kDense, MT>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, pf::kLds<MT>);
   });
   const int ncol = max_tiles ? H / (32 * pf::kWaves) : 0;
-  hipLaunchKernelGGL((moe_pf_down_kernel<FMT, kDense>), pf_grid(ncol, max_tiles, D), dim3(64 * pf::kWaves), pf::kLds,
+  hipLaunchKernelGGL((moe_pf_down_kernel<FMT, kDense, MT>), pf_grid(ncol, max_tiles, D), dim3(64 * pf::kWaves), pf::kLds<MT>,
                      s, d, ws, ws.act, routes, I, ws.y, H, ncol, D);
 }
 
-int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int max_tiles,
+int launch_moe_prefill_gate_up(int fmt, const Proj& g, const Proj& u, const MoeWs& ws, int mtile, int max_tiles,
                                const uint16_t* x, int B, int H, int I, const PfDense& D, hipStream_t s,
                                void* gate_up_start, void* after_gate_up) {
   dispatch_pf_format(fmt, [&](auto fc) {
     constexpr int FMT = decltype(fc)::value;
     if (D.tiles)
-      pf_launch_gate_up<FMT, true>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
+      pf_launch_gate_up<FMT, true, pf::kM>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
+    else if (mtile == 64)
+      pf_launch_gate_up<FMT, false, 64>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
     else
-      pf_launch_gate_up<FMT, false>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
+      pf_launch_gate_up<FMT, false, pf::kM>(g, u, ws, max_tiles, x, B, H, I, D, s, gate_up_start, after_gate_up);
   });
   return Q6MOE_OK;
 }
 
-int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int max_tiles, int routes, int H, int I,
+int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int mtile, int max_tiles, int routes, int H, int I,
                             const PfDense& D, hipStream_t s) {
   dispatch_pf_format(fmt, [&](auto fc) {
     constexpr int FMT = decltype(fc)::value;
     if (D.tiles)
-      pf_launch_down<FMT, true>(d, ws, max_tiles, routes, H, I, D, s);
+      pf_launch_down<FMT, true, pf::kM>(d, ws, max_tiles, routes, H, I, D, s);
+    else if (mtile == 64)
+      pf_launch_down<FMT, false, 64>(d, ws, max_tiles, routes, H, I, D, s);
     else
-      pf_launch_down<FMT, false>(d, ws, max_tiles, routes, H, I, D, s);
+      pf_launch_down<FMT, false, pf::kM>(d, ws, max_tiles, routes, H, I, D, s);
   });
   return Q6MOE_OK;
 }

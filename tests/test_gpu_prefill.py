@@ -176,3 +176,23 @@ def test_tiled_q5_k_layers(device, down, hidden, inter):
                   qtype="Q5_K", down_qtype=down, bias_sigma=1.0, pack=False)
     got, _ = _run(L, device, mode=2)
     assert_moe_close(got, _oracle(L))
+
+
+@pytest.mark.parametrize("qtype,down,hidden,inter", [("Q6_K", "Q8_0", 512, 640), ("Q8_0", "Q6_K", 384, 256),
+                                                     ("Q4_K", "Q5_1", 512, 384), ("Q5_K", "Q5_K", 256, 256)])
+def test_thin_tiles_of_every_width(device, qtype, down, hidden, inter):
+    # Up to 48 routes per expert on average the tiles hold 64 routes: experts of
+    # every column-group count, of exact multiples of 64 and one past them, and
+    # idle ones, in every format.
+    counts = [1, 31, 32, 33, 63, 64, 65, 128, 129, 0, 0, 0]
+    experts, tokens = len(counts), sum(counts)
+    assert tokens <= 48 * experts
+    L = moe_layer(seed=hidden, experts=experts, top_k=1, hidden=hidden, intermediate=inter, tokens=tokens,
+                  qtype=qtype, down_qtype=down, pack=False)
+    ids = np.random.default_rng(9).permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    got, _ = _run(L, device, mode=2, ids=ids)
+    assert_moe_close(got, _oracle(L, ids=ids))
+    # the same tokens twice (over 48 routes per expert: tiles of 128)
+    L2 = dict(L, x=np.concatenate([L["x"]] * 2), weights=np.concatenate([L["weights"]] * 2))
+    twice, _ = _run(L2, device, mode=2, ids=np.concatenate([ids] * 2))
+    np.testing.assert_array_equal(twice, np.concatenate([got, got]))
