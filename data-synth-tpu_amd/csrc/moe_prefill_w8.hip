@@ -221,6 +221,11 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 3)
   switch ((T.nv + 15) >> 4) {
     case 1: run(std::integral_constant<int, 1>{}); break;
     case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3:
+      if constexpr (PAIR) {  // its own width costs the down kernel spills that outweigh it
+        run(std::integral_constant<int, 3>{});
+        break;
+      }
     default: run(std::integral_constant<int, 4>{}); break;
   }
 }
