@@ -1420,15 +1420,39 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
               "tokens*top_k*max(hidden, intermediate, shared_intermediate) < 2^30");
     return Q6MOE_ERR_INVALID;
   }
+  const int fmt = fmt_of(a->gate.qtype), fmt_dn = fmt_of(a->down.qtype);
+  // The tiled MFMA kernels address token rows with 32-bit byte offsets.
+  const bool rows32 = B * H * 2 < (1ll << 31) && B * K * I * 2 < (1ll << 31);
+  const bool sh32 = B * H * 2 < (1ll << 31) && B * Is * 2 < (1ll << 31);
+  const bool sh_tiled_gu = Is && sh32 && pf_gate_up_supported(fmt, H, Is);
+  const bool sh_tiled_dn = Is && sh32 && pf_down_supported(fmt_dn, H, Is);
   // Mode 0: the decode-step kernels up to 64 tokens, unless the routing is
   // large (tokens x top-k x experts >= 2^17) and no shared expert rides along:
   // every decode-step wave repeats the routing over all entries and experts,
-  // and there the grouped kernels (routing once) are faster. Measured on the
-  // 512-expert top-10 layer: 16 tokens decode 141 us against grouped 158,
-  // 32 tokens 245 against 230, 64 tokens 432 against 345; the 128-expert
-  // top-8 layer at 64 tokens 125 against 124.
+  // and an expert's (and the shared expert's) weights are decoded again for
+  // every 16 of its tokens. Where the tiled kernels take the layer and its
+  // experts' row blocks alone fill the chip (experts x blocks >= 1024), the
+  // grouped kernels are faster from 2^16 on, from 2.5 routes per expert, and
+  // with a shared expert above 48 tokens. Measured (us, decode against grouped;
+  // even and skewed loads): 512-expert top-10 Q6_K/Q8_0 layer, 12 tokens 114 and
+  // 118, 97 and 105; 16 tokens 139 and 138, 123 and 119; 32 tokens 240 and 210,
+  // 197 and 171. 128-expert top-8 Q6_K layer, 32 tokens 107 and 104, 88 and 89;
+  // 40 tokens 111 and 107, 99 and 92; 64 tokens 124 and 112, 123 and 101; its
+  // Q5_K/Q8_0 form, 40 tokens 123 and 126, 113 and 109; 64 tokens 138 and 130,
+  // 136 and 116. 64-expert top-6 Q4_K layer with a shared expert, 40 tokens 133
+  // and 148, 132 and 125; 48 tokens 138 and 148, 145 and 127; 64 tokens 151 and
+  // 148, 180 and 135. The workspace bound keeps the choice the same for the
+  // entry point on the static scratch, and no call is refused for it.
   const bool dec_auto = B <= 64 && (Is > 0 || B * K * E < (int64_t(1) << 17));
-  const bool decode = !w8 && dec_supported(B, K, E, width) && (a->mode == 1 || (a->mode == 0 && dec_auto));
+  const auto group_few = [&] {
+    if (!rows32 || !pf_gate_up_supported(fmt, H, I) || !pf_down_supported(fmt_dn, H, I) || E * (I / 64) < 1024)
+      return false;
+    if (Is ? B <= 48 || !sh_tiled_gu || !sh_tiled_dn : B * K * E < (1 << 16) && 2 * B * K < 5 * E) return false;
+    const size_t need = ws_layout(B, K, E, H, I, Is, kPrefillTile, false).total;
+    return need <= kStaticScratchBytes && need <= workspace_bytes;
+  };
+  const bool decode = !w8 && dec_supported(B, K, E, width) &&
+                      (a->mode == 1 || (a->mode == 0 && dec_auto && !group_few()));
   const WsLayout L = ws_layout(B, K, E, H, I, Is, kPrefillTile, decode);
   if (workspace_bytes < L.total) {
     if (static_ws)
@@ -1472,7 +1496,6 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   auto mark = [&](int i) {
     if (a->events && a->events[i]) (void)hipEventRecord((hipEvent_t)a->events[i], s);
   };
-  const int fmt = fmt_of(a->gate.qtype), fmt_dn = fmt_of(a->down.qtype);
   // The shared expert outside the decode launches. Its gate/up and down run
   // tiled where the shape allows (full tiles of 128 tokens against blocks of
   // its rows), in the routed experts' launches where those are tiled too: its
@@ -1481,9 +1504,6 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   // 64 tokens. 64-expert top-6 Q4_K layer (H 4096, I 1024, shared 4096): at
   // 1024 tokens 868 us of generic kernels against 144 us more in the tiled
   // launches (the step 1150 -> 379 us); at 100 tokens 107 us against 23 us.
-  const bool sh32 = B * H * 2 < (1ll << 31) && B * Is * 2 < (1ll << 31);
-  const bool sh_tiled_gu = Is && sh32 && pf_gate_up_supported(fmt, H, Is);
-  const bool sh_tiled_dn = Is && sh32 && pf_down_supported(fmt_dn, H, Is);
   const Proj sg = make_proj(a->shared_gate, (int)Is, (int)H), su = make_proj(a->shared_up, (int)Is, (int)H),
              sd = make_proj(a->shared_down, (int)H, (int)Is);
   const TokenSrc dense{1, (int)B, nullptr, nullptr, nullptr, nullptr};
@@ -1558,8 +1578,6 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   }
   // int8_q8 policy: the Q8_0 projections run W8A8 (compute.py:20-34)
   const bool w8_gu = w8 && fmt == FMT_Q8, w8_dn = w8 && fmt_dn == FMT_Q8;
-  // The tiled MFMA kernels address token rows with 32-bit byte offsets.
-  const bool rows32 = B * H * 2 < (1ll << 31) && B * K * I * 2 < (1ll << 31);
   const bool tiled_gu = !w8_gu && rows32 && pf_gate_up_supported(fmt, H, I);
   const bool tiled_dn = !w8_dn && rows32 && pf_down_supported(fmt_dn, H, I);
   // the shared expert's items in the routed launches

@@ -588,3 +588,49 @@ def test_shared_gate_of_every_path(device, tokens, mode):
     want = fn(*tabs, x, ids, w, shared=dict(sh, scale=scale))
     assert (got == want).float().mean() > 0.99  # a sigmoid an ulp off may round its token's gate the other way
     np.testing.assert_allclose(got.float().cpu().numpy(), want.float().cpu().numpy(), rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("tokens,experts,top_k,shared,grouped", [
+    (39, 128, 8, 0, False), (40, 128, 8, 0, True),      # 2.5 routes per expert
+    (15, 512, 8, 0, False), (16, 512, 8, 0, True),      # tokens x top-k x experts of 2^16
+    (64, 64, 8, 0, False),                              # experts x row blocks below 1024
+    (48, 128, 4, 256, False), (49, 128, 4, 256, True),  # with a shared expert above 48 tokens
+    (64, 128, 4, 96, False),                            # whose shape the tiled kernels do not take
+])
+def test_default_family_by_size(device, tokens, experts, top_k, shared, grouped):
+    # Both families run every one of these calls; the default one gives the bits
+    # of the family that its rule names, in a Q4_K layer, where the families' sums
+    # differ in order.
+    rng = np.random.default_rng(tokens)
+    H, I = 1024, 512
+
+    def table(n, rows, width):
+        raw = rng.integers(0, 256, (n, rows, width // 256, 144), dtype=np.uint8)
+        d = rng.uniform(0.0001, 0.0002, (n, rows, width // 256, 1))
+        raw[..., :4] = np.concatenate([d, 7.5 * d], -1).astype(np.float16).view(np.uint8)  # centred weights
+        return raw.reshape(n, -1)
+
+    down = "Q8_0" if shared % 256 else "Q4_K"
+    fn = expert_parallel(None, gate_type="Q4_K", up_type="Q4_K", down_type=down, hidden=H, intermediate=I)
+
+    def down_table(n, width):
+        if down == "Q4_K":
+            return table(n, H, width)
+        raw = rng.integers(0, 256, (n, H, width // 32, 34), dtype=np.uint8)
+        raw[..., :2] = np.array([0.001], np.float16).view(np.uint8)
+        return raw.reshape(n, -1)
+
+    tabs = fn.prepare(table(experts, I, H), table(experts, I, H), down_table(experts, I), device)
+    sh = None
+    if shared:
+        sh = dict(gate=pack_experts(table(1, shared, H), "Q4_K", shared, H, device),
+                  up=pack_experts(table(1, shared, H), "Q4_K", shared, H, device),
+                  down=pack_experts(down_table(1, shared), down, H, shared, device))
+    torch.manual_seed(tokens)
+    x = torch.randn(tokens, H, device=device).to(torch.bfloat16)
+    ids = torch.rand(tokens, experts, device=device).topk(top_k).indices.to(torch.int32)
+    w = torch.rand(tokens, top_k, device=device).to(torch.bfloat16)
+    got, dec, grp = (fn.with_mode(m)(*tabs, x, ids, w, shared=sh) for m in (0, 1, 2))
+    assert torch.equal(got, grp if grouped else dec)
+    scale = dec.float().abs().max()
+    assert ((dec.float() - grp.float()).abs().max() / scale) < 1e-2
