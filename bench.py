@@ -716,7 +716,7 @@ def measure_prefill(dev, steps, warmup, with_cpu, down_qtype="Q6_K"):
         "mfma_fraction": round(tflops / MFMA_PEAK_TFLOPS, 4), "flops_per_step": PREFILL_FLOPS,
         "step_us": t["fused"],
         "phases_us": {k: round(float(v), 1) for k, v in zip(("route", "gate_up", "down", "combine"), ph)},
-        "roofline": roofline("q6moe::moe_pf_gate_up_kernel<0>", "mfma", PREFILL_FLOPS * 2 / 3, ph[1],
+        "roofline": roofline("q6moe::moe_pf_gate_up_kernel<0, false, 128>", "mfma", PREFILL_FLOPS * 2 / 3, ph[1],
                              work_unit="flops_per_launch", tag="4096 tokens"),
         "down_roofline": roofline(f"q6moe::moe_pf_down_kernel<{PF_FORMAT_ID[down_qtype]}>", "mfma",
                                   PREFILL_FLOPS / 3, ph[2], work_unit="flops_per_launch", tag="4096 tokens"),
@@ -798,7 +798,9 @@ def measure_q4_shared(dev, with_cpu):
                                   zip(("pre", "gate_up", "down", "combine") if b <= 64 else
                                       ("shared", "routed_gate_up", "routed_down", "combine"), ph)},
                     "active_experts": active, "bytes_per_step": nbytes, "layer_copies": want_copies,
-                    "roofline": roofline("q6moe::moe_dec_gate_up_kernel<1, true>", "hbm", gu_bytes, ph[1],
+                    # above 48 tokens the layer runs on the grouped kernels
+                    "roofline": roofline("q6moe::moe_dec_gate_up_kernel<1, true>" if b <= 48 else
+                                         "q6moe::moe_pf_gate_up_kernel<1, true, 128>", "hbm", gu_bytes, ph[1],
                                          work_unit="bytes_per_launch", tag=f"{b} token")})
         out["batches"][str(b)] = row
     return out
@@ -880,9 +882,9 @@ def measure_wide_layer(dev, with_cpu):
             layers.append(clone_tables(base))
         x, ids, w = xa[:b].contiguous(), ida[:b].contiguous(), wa[:b].contiguous()
         # the operator's default family (mode 0): the decode-step kernels, or
-        # the grouped ones once tokens x top-k x experts reaches 2^17
+        # the grouped ones once tokens x top-k x experts reaches 2^16
         f = fn
-        family = "grouped" if b * WIDE_K * WIDE_E >= 1 << 17 else "decode"
+        family = "grouped" if b * WIDE_K * WIDE_E >= 1 << 16 else "decode"
         ws = torch.empty(f.workspace_bytes(b, WIDE_K, WIDE_E), dtype=torch.uint8, device=dev)
         o = torch.empty((b, WIDE_H), dtype=torch.bfloat16, device=dev)
 
@@ -911,7 +913,7 @@ def measure_wide_layer(dev, with_cpu):
         # whose span the gate/up phase then measures: its bytes are the whole
         # step's but the combine's.
         fused = family == "decode" and 5 * b * WIDE_K < 2 * WIDE_E and b >= 8
-        kernel = ("q6moe::moe_pf_gate_up_kernel<0>" if family == "grouped" else
+        kernel = ("q6moe::moe_pf_gate_up_kernel<0, false, 64>" if family == "grouped" else
                   "q6moe::moe_dec_fused_kernel<0, 2, false>" if fused else "q6moe::moe_dec_gate_up_kernel<0, false>")
         if fused:
             gu_bytes += active * WIDE_DOWN_BYTES + routes * WIDE_H * 4

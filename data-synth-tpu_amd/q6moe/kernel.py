@@ -3,7 +3,8 @@
 Mirrors kaggle/packed_q6/kernel.py:98-148: same signature, argument checks
 and messages, FP32 result of ``x @ decode(W).T`` with BF16 operands and FP32
 accumulation, zero-padding of partial K blocks. The work is one launch of the
-HIP kernel ``q6_skinny_kernel`` (libq6moe.so); nothing runs on the CPU.
+HIP kernel ``q6_skinny_kernel`` (few tokens) or ``q6_tile_kernel`` (libq6moe.so);
+nothing runs on the CPU.
 
 ``batch_tile`` is validated as in the reference but does not change the
 result (the HIP kernel tiles tokens by 16). ``interpret`` is accepted for
