@@ -407,9 +407,9 @@ static int attn_pv_tiles(int64_t B, int64_t kvh, int64_t cap) {
   return tiles;
 }
 
-static AttnLayout attn_layout(int64_t B, int64_t hq, int64_t kvh, int64_t cap) {
+static AttnLayout attn_layout(int64_t B, int64_t hq, int64_t kvh, int64_t cap, int pv_tiles) {
   AttnLayout L;
-  const int64_t nchunks = cdiv(cap, attn_pv_tiles(B, kvh, cap) * kPvThreads);
+  const int64_t nchunks = cdiv(cap, pv_tiles * kPvThreads);
   L.s = 0;
   L.wstats = attn_align(L.s + (size_t)B * hq * cap * 2);
   L.part = attn_align(L.wstats + (size_t)B * hq * (cap / kAttnWaveTok) * 2 * 4);
@@ -424,7 +424,8 @@ using namespace q6moe;
 extern "C" size_t q6moe_attn_workspace_size(int64_t batch, int64_t query_heads, int64_t kv_heads,
                                             int64_t pages_per_seq, int64_t page_size) {
   if (batch < 1 || query_heads < 1 || kv_heads < 1 || pages_per_seq < 1 || page_size < 1) return 0;
-  return attn_layout(batch, query_heads, kv_heads, pages_per_seq * page_size).total;
+  const int64_t cap = pages_per_seq * page_size;
+  return attn_layout(batch, query_heads, kv_heads, cap, attn_pv_tiles(batch, kv_heads, cap)).total;
 }
 
 extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream) {
@@ -445,7 +446,11 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   Q6MOE_REQUIRE(aligned(a->q, 16) && aligned(a->k_codes, 16) && aligned(a->v_codes, 16) && aligned(a->out, 4) &&
                     aligned(a->workspace, 256),
                 "decode_attention: q/codes need 16-byte, out 4-byte and workspace 256-byte alignment");
-  const AttnLayout L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap);
+  // a workspace too small for the narrower chunks' partial sums still takes the wider ones
+  int tiles = attn_pv_tiles(a->batch, a->kv_heads, cap);
+  AttnLayout L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap, tiles);
+  while (a->workspace_bytes < L.total && tiles < kPvMaxTiles)
+    L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap, tiles *= 2);
   if (a->workspace_bytes < L.total) {
     set_error("decode_attention: workspace too small (need " + std::to_string(L.total) + " bytes)");
     return Q6MOE_ERR_INVALID;
@@ -465,7 +470,7 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   p.hq = (int)a->query_heads;
   p.r = (int)(a->query_heads / a->kv_heads);
   p.cap = (int)cap;
-  p.pv_tiles = attn_pv_tiles(a->batch, p.kvh, cap);
+  p.pv_tiles = tiles;
   p.nchunks = (int)cdiv(cap, p.pv_tiles * kPvThreads);
   uint8_t* w = reinterpret_cast<uint8_t*>(a->workspace);
   p.s = reinterpret_cast<uint16_t*>(w + L.s);

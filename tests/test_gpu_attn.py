@@ -146,3 +146,31 @@ def test_decode_attention_chunk_widths(device, batch, kvh, pps, lengths):
     for lens in lengths:
         got, qv = _run(device, pools, scales, table, q, lens, page_size, kvh)
         _check(got[rows], _want(pools, scales, table, qv, lens, page_size, kvh, rows=rows))
+
+
+def test_decode_attention_takes_a_workspace_of_the_wider_chunks(device, monkeypatch):
+    # 512-token chunks ask for more partial sums; a workspace that holds those of
+    # 2048-token chunks is still taken, a smaller one refused
+    from q6moe import _lib, attention_cache
+
+    pools, scales, table, q = _case(31, 1, 2, 4, pages=66, page_size=64, pps=64)
+    lengths, cap = [4000], 4096
+    args = [torch.from_numpy(t).to(device) for t in (pools[0], scales[0], pools[1], scales[1], table)]
+    qt = torch.from_numpy(q).to(device).to(torch.bfloat16)
+    lens = torch.tensor(lengths, dtype=torch.int32, device=device)
+
+    def need(chunk):  # scores, statistics per 64 tokens, partial sums
+        up = lambda n: -(-n // 256) * 256  # noqa: E731
+        return up(8 * cap * 2) + up(8 * (cap // 64) * 8) + up(2 * (cap // chunk) * 8 * 128 * 4)
+
+    def run(nbytes):
+        monkeypatch.setattr(attention_cache, "_attn_workspace_bytes", lambda *a: nbytes)
+        return paged_decode_attention(qt, *args, lens, page_size=64, kv_heads=2)
+
+    assert int(_lib.load().q6moe_attn_workspace_size(1, 8, 2, 64, 64)) == need(512)
+    outs = [run(need(c)).float().cpu().numpy() for c in (512, 1024, 2048)]
+    want = _want(pools, scales, table, qt.float().cpu().numpy(), lengths, 64, 2)
+    for got in outs:
+        _check(got, want)
+    with pytest.raises(_lib.Q6MoeError, match="workspace too small"):
+        run(need(2048) - 256)
