@@ -1,8 +1,10 @@
 // W8A8 policy of Q8_0 projections on the INT8 matrix cores, tiled: the rows of
 // kaggle/qwen38_tpu/compute.py:20-34 (q8_matmul) for routed tiles of tokens.
 // Per 32-value group one v_mfma_i32_16x16x32_i8 gives exact INT32 dot products
-// p; the result is sum over groups, in order, of fma(f32(p) * s_x, d_w) in
-// FP32, rounded to BF16.
+// p; a 256-wide K block's sum is fma(f32(p) * s_x, d_w) over its groups, in
+// order, in FP32, and the result is the sum of the K blocks, in order, rounded to
+// BF16: the order of moe_w8_kernel's waves (one block each up to 2048 inputs), so
+// that the number of tokens does not show, and no chain is longer than its own.
 //
 // Bound by the vector ALU: each partial product takes a conversion, a multiply
 // by the token's scale and a fused multiply-add by the row's (v_fma_mix_f32,
@@ -12,11 +14,15 @@
 // 256-wide K block) per K block, whose codes and scales it loads straight into
 // registers in MFMA layout; the routes' codes (16 KB per K block, XOR-swizzled
 // so that an operand read touches every bank once) and scales are
-// double-buffered in LDS by direct buffer->LDS DMA. 64 routes rather than the
-// tile's 128 keep the accumulators and one weight set within 168 registers, so
-// three waves share a SIMD and the conversions issue back to back. Against the
-// kernel of 16 tokens per weight pass (moe_w8_kernel), 128-expert top-8 layer,
-// H 2048, I 768, 1024 tokens: gate/up 1473 -> 181 us, down 1075 -> 100 us.
+// double-buffered in LDS by direct buffer->LDS DMA. The running and the K block's
+// sums take 64 registers, so two waves share a SIMD (212 registers; held to 168
+// for a third, the kernel spills and takes 295-570 us for the step below that
+// takes 291): four groups' MFMAs go first, then their conversions, products and
+// sums, eight independent instructions at a time, since with two waves nothing
+// else covers a dependent one's wait (306 -> 291 us). 128-expert top-8 layer,
+// H 2048, I 768, 1024 tokens, cold weights: gate/up 1473 us by the kernel of 16
+// tokens per weight pass (moe_w8_kernel), 189 us here, down 1075 and 108 (one
+// chain over K at three waves per SIMD: 175 and 98 us).
 #include "moe_tile.h"
 #include "q6moe_api.h"
 
@@ -119,23 +125,45 @@ __device__ __forceinline__ void w8_stream(uint8_t* smem, const uint8_t* const (&
     if (more) dma(kb + 1);
     const uint8_t* st = smem + (kb & 1) * kW8Stage;
     const int ng = groups - 8 * kb;
+    f32x4 blk[kUnits][NCG];
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+      for (int t = 0; t < NCG; ++t) blk[u][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     static_for<0, 2>([&](auto qc) {
       constexpr int quad = decltype(qc)::value;
       if (4 * quad < ng) {  // false only in the second half of a last, half K block
 #pragma unroll
         for (int tg = 0; tg < NCG; ++tg) {
           const f32x4 sa = *reinterpret_cast<const f32x4*>(st + kW8Codes + (tg * 16 + j) * 32 + 16 * quad);
+          // this column group's 8 MFMAs first, then their conversions, so that none waits for its product
+          i32x4 p[4][kUnits];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const int G = 4 * quad + q;
             const uint64_t b = *reinterpret_cast<const uint64_t*>(st + xgran(tg * 16 + j, 2 * G + (kq >> 1)) + 8 * (kq & 1));
 #pragma unroll
-            for (int u = 0; u < kUnits; ++u) {
-              const i32x4 p = mfma_i8z(w[u].c[G], b);
+            for (int u = 0; u < kUnits; ++u) p[q][u] = mfma_i8z(w[u].c[G], b);
+          }
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                acc[u][tg][i] = __builtin_fmaf((float)p[i] * sa[q], w[u].scale(i, G), acc[u][tg][i]);
-            }
+          for (int q = 0; q < 4; ++q) {
+            float v[kUnits][4];
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[u][i] = (float)p[q][u][i];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) v[u][i] *= sa[q];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) blk[u][tg][i] = __builtin_fmaf(v[u][i], w[u].scale(i, 4 * quad + q), blk[u][tg][i]);
+            __builtin_amdgcn_sched_barrier(0);
           }
         }
       }
@@ -151,6 +179,10 @@ __device__ __forceinline__ void w8_stream(uint8_t* smem, const uint8_t* const (&
       }
       __builtin_amdgcn_sched_barrier(0);
     });
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u)
+#pragma unroll
+      for (int t = 0; t < NCG; ++t) acc[u][t] += blk[u][t];
   }
 }
 
@@ -162,7 +194,7 @@ __device__ __forceinline__ void w8_stream(uint8_t* smem, const uint8_t* const (&
 // row of a route: its token (gate/up) or its position (``route_rows``, down);
 // dense items (D.tiles > 0, p0 only): the token.
 template <bool PAIR>
-__global__ void __launch_bounds__(64 * pf::kWaves, 3)
+__global__ void __launch_bounds__(64 * pf::kWaves, 2)
     moe_pf_w8_kernel(Proj p0, Proj p1, MoeWs ws, int route_rows, W8Src a, int a_rows, uint16_t* __restrict__ out,
                      int ncol, PfDense D) {
   using namespace pf;
@@ -221,11 +253,7 @@ __global__ void __launch_bounds__(64 * pf::kWaves, 3)
   switch ((T.nv + 15) >> 4) {
     case 1: run(std::integral_constant<int, 1>{}); break;
     case 2: run(std::integral_constant<int, 2>{}); break;
-    case 3:
-      if constexpr (PAIR) {  // its own width costs the down kernel spills that outweigh it
-        run(std::integral_constant<int, 3>{});
-        break;
-      }
+    case 3: run(std::integral_constant<int, 3>{}); break;
     default: run(std::integral_constant<int, 4>{}); break;
   }
 }

@@ -163,3 +163,16 @@ def test_int8_q8_tiles_of_every_width(device, hidden, inter):
                                  hidden=hidden, intermediate=inter, policy="int8_q8")
     assert_moe_close(got, want)
     np.testing.assert_array_equal(got, fn(*args).float().cpu().numpy())
+
+
+@pytest.mark.parametrize("k", [128, 1152, 2048])
+def test_q8_matmul_sums_in_the_same_order_at_every_token_count(device, k):
+    # Up to 64 tokens eight waves split K, one 256-wide block each here, and their
+    # sums meet in block order; the tiled kernel sums its K blocks apart in the
+    # same order, so up to 2048 inputs a token's result does not depend on how many
+    # others there are, bit for bit (one chain over K differs in 1e-4 of the values).
+    rng = np.random.default_rng(k)
+    packed = torch.from_numpy(pack_q8(rng.normal(0, 0.05, (1024, k)).astype(np.float32))).to(device)
+    x = torch.from_numpy(rng.normal(size=(192, k)).astype(np.float32)).to(device).to(torch.bfloat16)
+    parts = torch.cat([q8_matmul(x[i: i + 64].contiguous(), packed) for i in (0, 64, 128)])
+    assert torch.equal(q8_matmul(x, packed), parts)
