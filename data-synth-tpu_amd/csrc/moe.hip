@@ -1749,11 +1749,13 @@ extern "C" int q6moe_q8_matmul(const uint16_t* x, int64_t m, int64_t k, const ui
   q6moe_table t{Q6MOE_Q8_0, table, (int64_t)unit_table_bytes(Q6MOE_Q8_0, n, k), nullptr, 0};
   const Proj p = make_proj(t, (int)n, (int)k);
   const W8Src src{codes, scales, (int)k};
-  // Tiled above 64 tokens (64-token tiles, no K split); below, splitting K over
-  // 8 waves gives the few row groups more waves. 4096 x 4096: 64 tokens 46.7 us
-  // split, 59.5 tiled; 128 tokens 88.9 and 60.4; 640 x 2560: 35.5 and 37.7, 66.0
-  // and 37.9.
-  if (m > 64 && m * k < (1ll << 31) && aligned(y, 8) && pf_w8_supported(false, n, k)) {
+  // Tiled above 64 tokens (64-token tiles, no K split), above 72 for more than 12
+  // K blocks, which pass one after another; below, splitting K over 8 waves gives
+  // the few row groups more waves. Split and tiled (us): 4096 x 4096 (rows x
+  // inputs), 65 tokens 51.8 and 53.7, 73 tokens 54.9 and 53.6; 1024 x 16384, 65
+  // tokens 179 and 192, 73 tokens 191 and 193, 76 tokens 196 and 193; 2560 x 3072,
+  // 65 tokens 43.5 and 39.6; 640 x 2560, 48 tokens 28.1 split, 65 tokens 39.8 and 34.1.
+  if (m > (k > 12 * kQK ? 72 : 64) && m * k < (1ll << 31) && aligned(y, 8) && pf_w8_supported(false, n, k)) {
     launch_prefill_w8_dense(p, src, (int)m, y, s);
   } else {
     TokenSrc dense{1, (int)m, nullptr, nullptr, nullptr, nullptr};
