@@ -17,15 +17,15 @@
 //      channels per v_mfma_f32_16x16x32_bf16) against the group's query
 //      heads as B operand; scores go to the workspace as BF16, and each
 //      wave's maximum m_w and sum l_w of exp(score - m_w) over its 64 tokens.
-//   2. attn_pv_kernel: per 2048-token chunk (8 waves, four 64-token tiles
-//      each; 1024 or 512 tokens for few sequences), wave h first merges head h's statistics over the attended
-//      tokens, max = max_w m_w and sum = sum_w l_w exp(m_w - max) in a fixed
-//      order; the workgroup forms RNE_bf16(prob) once per (head, token) in
-//      LDS; each wave then runs P.V for its tiles, in turn, on MFMA with the
-//      dequantised values as A operand (row = 8 channels apart, so a lane
-//      dequantises the 8x8 code block it loaded straight into eight tiles'
-//      operands) and the probabilities as B; the chunk's partial sums go to
-//      the workspace.
+//   2. attn_pv_kernel: per 2048-token chunk (8 waves, four 64-token tiles each;
+//      1024 or 512 tokens for few sequences), wave h first merges head h's
+//      statistics over the attended tokens, max = max_w m_w and sum = sum_w l_w
+//      exp(m_w - max) in a fixed order; the workgroup forms RNE_bf16(prob) once
+//      per (head, token) in LDS; each wave then runs P.V for its tiles, in turn,
+//      on MFMA with the dequantised values as A operand (row = 8 channels apart,
+//      so a lane dequantises the 8x8 code block it loaded straight into eight
+//      tiles' operands) and the probabilities as B; the chunk's partial sums go
+//      to the workspace (a narrower chunk's in place of its scores).
 //   3. attn_combine_kernel: partial sums over chunks in a fixed order, RNE.
 //
 // HBM-bound: the INT8 codes and scales of K and V are read once.
@@ -51,11 +51,11 @@ struct AttnParams {
   const int32_t* table;              // [B, pps]
   const int32_t* len;                // [B]
   int64_t pool_pages;
-  int pps, page, kvh, hq, r, cap, nchunks;  // nchunks: P.V chunks of pv_tiles * kPvThreads tokens
-  int pv_tiles;
+  int pps, page, kvh, hq, r, cap, nchunks;  // nchunks: P.V chunks of kPvMaxTiles * kPvThreads tokens
+  int pv_tiles;                             // of this call: chunks of pv_tiles * kPvThreads tokens
   uint16_t* s;                       // [B, Hq, cap] BF16 scores
   float* wstats;                     // [B, Hq, cap / 64, 2]: per 64 tokens, max m_w and sum of exp(score - m_w)
-  float* part;                       // [B, KVH, nchunks, kAttnR, D]
+  float* part;                       // [B, KVH, nchunks, kAttnR, D]; narrower chunks: [B, Hq, D]
   uint16_t* out;                     // [B, Hq, D]
 };
 
@@ -178,6 +178,16 @@ __global__ void __launch_bounds__(256) attn_scores_kernel(AttnParams p) {
     float* ws = p.wstats + (((int64_t)b * p.hq + kh * p.r + col) * (p.cap / kAttnWaveTok) + t0 / kAttnWaveTok) * 2;
     *reinterpret_cast<f32x2*>(ws) = f32x2{m, l};
   }
+}
+
+// The partial sum of head h (of sequence b) over the chunk at token c0 where the
+// chunks are narrower than the widest: it takes the place of the chunk's first
+// 256 scores, which only the workgroup that writes it reads, and has read by
+// then; a last chunk of fewer tokens writes to ``part``. So the workspace is that
+// of the widest chunks at every size of a call.
+__device__ __forceinline__ float* attn_narrow_part(const AttnParams& p, int b, int h, int c0) {
+  const int64_t row = (int64_t)b * p.hq + h;
+  return c0 + 2 * kAttnD <= p.cap ? reinterpret_cast<float*>(p.s + row * p.cap + c0) : p.part + row * kAttnD;
 }
 
 template <int kPvTiles>
@@ -352,12 +362,16 @@ __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu
   }
   __syncthreads();
   float* dst = p.part + (((int64_t)b * p.kvh + kh) * p.nchunks + chunk) * kAttnR * kAttnD;
-  for (int o = threadIdx.x; o < kAttnR * kAttnD; o += kPvThreads) {
+  const int heads = kPvTiles == kPvMaxTiles ? kAttnR : p.r;
+  for (int o = threadIdx.x; o < heads * kAttnD; o += kPvThreads) {
     const int h = o / kAttnD, d = o % kAttnD;
     float v = red[0][h][d];
 #pragma unroll
     for (int w = 1; w < kPvWaves; ++w) v += red[w][h][d];
-    dst[o] = v;
+    if constexpr (kPvTiles == kPvMaxTiles)
+      dst[o] = v;
+    else
+      attn_narrow_part(p, b, kh * p.r + h, c0)[d] = v;
   }
 }
 
@@ -371,11 +385,15 @@ __global__ void __launch_bounds__(8 * kAttnD) attn_combine_kernel(AttnParams p) 
   const int nc = (attn_len(p, b) + pv_chunk - 1) / pv_chunk;
   const int per = (nc + 7) / 8, cb = grp * per, ce = cb + per < nc ? cb + per : nc;
   const float* src = p.part + (((int64_t)b * p.kvh + kh) * p.nchunks) * kAttnR * kAttnD + hr * kAttnD + d;
+  const auto part = [&](int c) {
+    return p.pv_tiles == kPvMaxTiles ? src[(int64_t)c * kAttnR * kAttnD]
+                                     : attn_narrow_part(p, b, h, c * pv_chunk)[d];
+  };
   float v = 0.f;
   for (int c0 = cb; c0 < ce; c0 += 8) {
     float x[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = c0 + u < ce ? src[(int64_t)(c0 + u) * kAttnR * kAttnD] : 0.f;
+    for (int u = 0; u < 8; ++u) x[u] = c0 + u < ce ? part(c0 + u) : 0.f;
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (c0 + u < ce) v += x[u];
@@ -407,9 +425,9 @@ static int attn_pv_tiles(int64_t B, int64_t kvh, int64_t cap) {
   return tiles;
 }
 
-static AttnLayout attn_layout(int64_t B, int64_t hq, int64_t kvh, int64_t cap, int pv_tiles) {
+static AttnLayout attn_layout(int64_t B, int64_t hq, int64_t kvh, int64_t cap) {
   AttnLayout L;
-  const int64_t nchunks = cdiv(cap, pv_tiles * kPvThreads);
+  const int64_t nchunks = cdiv(cap, kPvMaxTiles * kPvThreads);
   L.s = 0;
   L.wstats = attn_align(L.s + (size_t)B * hq * cap * 2);
   L.part = attn_align(L.wstats + (size_t)B * hq * (cap / kAttnWaveTok) * 2 * 4);
@@ -424,8 +442,7 @@ using namespace q6moe;
 extern "C" size_t q6moe_attn_workspace_size(int64_t batch, int64_t query_heads, int64_t kv_heads,
                                             int64_t pages_per_seq, int64_t page_size) {
   if (batch < 1 || query_heads < 1 || kv_heads < 1 || pages_per_seq < 1 || page_size < 1) return 0;
-  const int64_t cap = pages_per_seq * page_size;
-  return attn_layout(batch, query_heads, kv_heads, cap, attn_pv_tiles(batch, kv_heads, cap)).total;
+  return attn_layout(batch, query_heads, kv_heads, pages_per_seq * page_size).total;
 }
 
 extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream) {
@@ -446,11 +463,7 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   Q6MOE_REQUIRE(aligned(a->q, 16) && aligned(a->k_codes, 16) && aligned(a->v_codes, 16) && aligned(a->out, 4) &&
                     aligned(a->workspace, 256),
                 "decode_attention: q/codes need 16-byte, out 4-byte and workspace 256-byte alignment");
-  // a workspace too small for the narrower chunks' partial sums still takes the wider ones
-  int tiles = attn_pv_tiles(a->batch, a->kv_heads, cap);
-  AttnLayout L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap, tiles);
-  while (a->workspace_bytes < L.total && tiles < kPvMaxTiles)
-    L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap, tiles *= 2);
+  const AttnLayout L = attn_layout(a->batch, a->query_heads, a->kv_heads, cap);
   if (a->workspace_bytes < L.total) {
     set_error("decode_attention: workspace too small (need " + std::to_string(L.total) + " bytes)");
     return Q6MOE_ERR_INVALID;
@@ -470,8 +483,8 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   p.hq = (int)a->query_heads;
   p.r = (int)(a->query_heads / a->kv_heads);
   p.cap = (int)cap;
-  p.pv_tiles = tiles;
-  p.nchunks = (int)cdiv(cap, p.pv_tiles * kPvThreads);
+  p.pv_tiles = attn_pv_tiles(a->batch, a->kv_heads, cap);
+  p.nchunks = (int)cdiv(cap, kPvMaxTiles * kPvThreads);
   uint8_t* w = reinterpret_cast<uint8_t*>(a->workspace);
   p.s = reinterpret_cast<uint16_t*>(w + L.s);
   p.wstats = reinterpret_cast<float*>(w + L.wstats);
@@ -479,7 +492,7 @@ extern "C" int q6moe_kv_decode_attention(const q6moe_attn_args* a, void* stream)
   p.out = a->out;
   hipStream_t s = (hipStream_t)stream;
   const dim3 chunks((unsigned)((cap + kAttnChunk - 1) / kAttnChunk), (unsigned)p.kvh, (unsigned)a->batch);
-  const dim3 pv_chunks((unsigned)p.nchunks, (unsigned)p.kvh, (unsigned)a->batch);
+  const dim3 pv_chunks((unsigned)cdiv(cap, p.pv_tiles * kPvThreads), (unsigned)p.kvh, (unsigned)a->batch);
   hipLaunchKernelGGL(attn_scores_kernel, chunks, dim3(256), 0, s, p);
   if (p.pv_tiles == 4)
     hipLaunchKernelGGL(attn_pv_kernel<4>, pv_chunks, dim3(kPvThreads), 0, s, p);

@@ -148,29 +148,42 @@ def test_decode_attention_chunk_widths(device, batch, kvh, pps, lengths):
         _check(got[rows], _want(pools, scales, table, qv, lens, page_size, kvh, rows=rows))
 
 
-def test_decode_attention_takes_a_workspace_of_the_wider_chunks(device, monkeypatch):
-    # 512-token chunks ask for more partial sums; a workspace that holds those of
-    # 2048-token chunks is still taken, a smaller one refused
-    from q6moe import _lib, attention_cache
+@pytest.mark.parametrize("kvh,r,pps", [(4, 1, 128), (4, 8, 16), (2, 4, 33)])
+def test_one_workspace_serves_every_smaller_call(device, kvh, r, pps):
+    # a serving loop sizes its workspace for the largest batch and keeps it as
+    # sequences end: every smaller batch takes it, at every chunk width, with the
+    # results of a workspace of its own
+    from q6moe import _lib
 
-    pools, scales, table, q = _case(31, 1, 2, 4, pages=66, page_size=64, pps=64)
-    lengths, cap = [4000], 4096
-    args = [torch.from_numpy(t).to(device) for t in (pools[0], scales[0], pools[1], scales[1], table)]
+    size = _lib.load().q6moe_attn_workspace_size
+    pages, page_size, most = pps + 2, 64, 9
+    pools, scales, table, q = _case(5 + kvh, most, kvh, r, pages=pages, page_size=page_size, pps=pps)
+    args = [torch.from_numpy(t).to(device) for t in (pools[0], scales[0], pools[1], scales[1])]
     qt = torch.from_numpy(q).to(device).to(torch.bfloat16)
-    lens = torch.tensor(lengths, dtype=torch.int32, device=device)
+    tt = torch.from_numpy(table).to(device)
+    lengths = [pps * page_size - 37 * i for i in range(most)]
+    ws = torch.empty(int(size(most, kvh * r, kvh, pps, page_size)), dtype=torch.uint8, device=device)
+    for batch in range(most, 0, -1):
+        lens = torch.tensor(lengths[:batch], dtype=torch.int32, device=device)
+        call = lambda **kw: paged_decode_attention(qt[:batch], *args, tt[:batch], lens, page_size=page_size,  # noqa: E731
+                                                   kv_heads=kvh, **kw)
+        got = call(workspace=ws)
+        assert torch.equal(got, call())
+        exact = int(size(batch, kvh * r, kvh, pps, page_size))
+        assert torch.equal(got, call(workspace=ws[:exact]))
+        with pytest.raises(ValueError, match="workspace"):
+            call(workspace=ws[:exact - 1])
+        if batch in (1, 3):
+            want = _want(pools, scales, table[:batch], qt[:batch].float().cpu().numpy(), lengths[:batch], page_size, kvh)
+            _check(got.float().cpu().numpy(), want)
 
-    def need(chunk):  # scores, statistics per 64 tokens, partial sums
-        up = lambda n: -(-n // 256) * 256  # noqa: E731
-        return up(8 * cap * 2) + up(8 * (cap // 64) * 8) + up(2 * (cap // chunk) * 8 * 128 * 4)
 
-    def run(nbytes):
-        monkeypatch.setattr(attention_cache, "_attn_workspace_bytes", lambda *a: nbytes)
-        return paged_decode_attention(qt, *args, lens, page_size=64, kv_heads=2)
-
-    assert int(_lib.load().q6moe_attn_workspace_size(1, 8, 2, 64, 64)) == need(512)
-    outs = [run(need(c)).float().cpu().numpy() for c in (512, 1024, 2048)]
-    want = _want(pools, scales, table, qt.float().cpu().numpy(), lengths, 64, 2)
-    for got in outs:
-        _check(got, want)
-    with pytest.raises(_lib.Q6MoeError, match="workspace too small"):
-        run(need(2048) - 256)
+@pytest.mark.parametrize("pps,page_size", [(1, 64), (3, 64), (8, 64), (9, 64), (11, 64), (12, 64), (13, 128)])
+def test_decode_attention_narrow_chunks_at_the_end_of_the_capacity(device, pps, page_size):
+    # 512-token chunks: a last chunk of fewer than 256 tokens of capacity has no
+    # room for its partial sum among its scores
+    pools, scales, table, q = _case(9 + pps, 2, 2, 3, pages=20, page_size=page_size, pps=pps)
+    cap = pps * page_size
+    for lens in ([cap, cap - 1], [max(1, cap - 64), 1]):
+        got, qv = _run(device, pools, scales, table, q, lens, page_size, 2)
+        _check(got, _want(pools, scales, table, qv, lens, page_size, 2))

@@ -199,3 +199,21 @@ def test_score_scaling_by_the_reciprocal_is_exact_in_bf16():
         return (u + 0x7FFF + ((u >> 16) & 1)) >> 16
 
     np.testing.assert_array_equal(bf16(x / d), bf16(x * (np.float32(1) / d)))
+
+
+def test_attention_workspace_serves_every_smaller_call():
+    # scores, statistics per 64 tokens and partial sums per 2048 tokens, at every
+    # size of a call: never less for more sequences or pages
+    from q6moe import _lib
+
+    size = _lib.load().q6moe_attn_workspace_size
+
+    def need(batch, hq, kvh, cap):
+        up = lambda n: -(-n // 256) * 256  # noqa: E731
+        return up(batch * hq * cap * 2) + up(batch * hq * (cap // 64) * 8) + up(batch * kvh * -(-cap // 2048) * 4096)
+
+    for kvh, r in ((4, 1), (4, 8), (2, 1), (8, 1), (8, 6), (1, 3)):
+        for pps in (1, 4, 32, 33, 128, 512):
+            sizes = [int(size(b, kvh * r, kvh, pps, 64)) for b in range(1, 20)]
+            assert sizes == [need(b, kvh * r, kvh, pps * 64) for b in range(1, 20)]
+            assert sizes == sorted(sizes)
