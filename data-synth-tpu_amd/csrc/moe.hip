@@ -1582,15 +1582,24 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   const bool tiled_dn = !w8_dn && rows32 && pf_down_supported(fmt_dn, H, I);
   // the shared expert's items in the routed launches
   const bool join_gu = sh_tiled_gu && tiled_gu, join_dn = sh_tiled_dn && tiled_dn;
-  // Tiles of 64 routes up to 48 routes per expert on average: three waves per
-  // SIMD decode faster than the second 64 routes of a tile save. 512-expert
-  // top-10 Q6_K/Q8_0 layer, step: 200 tokens 475 us with 128 and 457 with 64,
-  // 2001 tokens 621 and 585; 128-expert top-8 layer: 128 tokens 132 and 124 us,
-  // 512 tokens 157 and 150, 768 (48 per expert) 168 and 168, 1024 183 and 195. Same
-  // outputs. Their more tile records take the place of the W8A8 policy's
+  // Tiles of 64 routes where the experts see few: with Q6_K and Q8_0 weights
+  // (pf_thin_dense) three waves per SIMD decode faster than the second 64 routes of
+  // a tile save, up to 48 routes per expert on average where every tiled
+  // projection is of these formats, up to 36 where one of the two is. The other
+  // formats gain no wave and decode an expert of more than 64 routes twice. Same
+  // outputs. 128-expert top-8 layer (H 2048, I 768), grouped step (us, tiles of 128
+  // and 64; even and skewed loads): Q6_K pair, 24 routes per expert 143.6 and 135.3,
+  // 154.3 and 143.3; 48 163.1 and 160.6, 178.3 and 170.9; Q8_0 pair, 24 155.4 and
+  // 151.1; 48 173.0 and 174.5, 187.4 and 182.9. Q4_K with Q8_0, 36 152.5 and 149.5,
+  // 161.1 and 160.2; 48 161.3 and 165.9; Q6_K with Q5_1, 36 154.9 and 150.3; 48
+  // 167.0 and 170.6. Q4_K pair, 16 116.5 and 116.9, 119.1 and 122.0; 48 148.5 and
+  // 156.0, 162.6 and 171.7; Q5_K pair, 16 142.9 and 141.8, 146.3 and 150.7; 48 174.1
+  // and 182.9. The 64-route tiles' more records take the place of the W8A8 policy's
   // buffers, unused here, where these are large enough.
+  const bool thin_all = (!tiled_gu || pf_thin_dense(fmt)) && (!tiled_dn || pf_thin_dense(fmt_dn));
+  const bool thin_any = (tiled_gu && pf_thin_dense(fmt)) || (tiled_dn && pf_thin_dense(fmt_dn));
   const int64_t thin_bytes = (int64_t)sizeof(PfTile) * (E + B * K / kThinTile + 1);
-  const bool thin = B * K <= 48 * E && !w8 && !join_gu && !join_dn && (tiled_gu || tiled_dn) &&
+  const bool thin = thin_any && B * K <= (thin_all ? 48 : 36) * E && !w8 && !join_gu && !join_dn &&
                     thin_bytes <= (int64_t)(L.total - L.xq);
   const int mtile = (int)(thin ? kThinTile : kPrefillTile);
   const int max_tiles = (int)(E + B * K / mtile + 1);

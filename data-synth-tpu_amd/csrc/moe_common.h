@@ -235,6 +235,9 @@ int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStre
 // Prefill grouped GEMM, tiled on the matrix cores: gate/up (every format but
 // Q5_1; hidden a multiple of 128, intermediate of 64) and down (every format;
 // intermediate a multiple of 128, hidden of 128), each launched on its own.
+// Tiles hold up to 128 routes, or 64: with these formats' weights three
+// workgroups of the 64-route kernels share a CU, with the others' two, as at 128.
+constexpr bool pf_thin_dense(int fmt) { return fmt == FMT_Q6 || fmt == FMT_Q8; }
 bool pf_gate_up_supported(int fmt, int64_t H, int64_t I);
 bool pf_down_supported(int fmt, int64_t H, int64_t I);
 // A dense expert (the always-on shared one: every token, weight 1) whose items

@@ -48,7 +48,7 @@ constexpr int kXStages = 2;        // token-tile stages in LDS: the K half being
 template <int MT>
 constexpr int kLds = kXStages * kHalfBytes<MT>;
 template <int FMT, int MT>
-constexpr int kWgPerCu = MT == 64 && (FMT == FMT_Q6 || FMT == FMT_Q8) ? 3 : 2;
+constexpr int kWgPerCu = MT == 64 && pf_thin_dense(FMT) ? 3 : 2;
 
 // The weights of one unit (a whole K block) in the registers of the lane that
 // decodes them (row j = lane % 16, k-group jA = lane / 16); both K halves

@@ -41,3 +41,27 @@ def test_q8_matmul_kernel_by_size(device, inputs, tokens, tiled):
     w = torch.from_numpy(q8_table(np.random.default_rng(1), 1, 256, inputs)[0]).to(device)
     x = torch.randn(tokens, inputs, device=device).to(torch.bfloat16)
     assert launched(lambda: q8_matmul(x, w), "moe_pf_w8_kernel") == tiled
+
+
+@pytest.mark.parametrize("qtype,down,most", [
+    ("Q6_K", "Q6_K", 48), ("Q8_0", "Q6_K", 48),                                         # both keep a third wave
+    ("Q4_K", "Q8_0", 36), ("Q6_K", "Q5_1", 36), ("Q5_K", "Q8_0", 36), ("Q6_K", "Q4_K", 36),  # one of them
+    ("Q4_K", "Q4_K", 0), ("Q5_K", "Q5_1", 0),                                           # neither
+])
+def test_tile_width_by_format_and_routes_per_expert(device, qtype, down, most):
+    from q6moe.experts import expert_parallel
+    from q6moe.synth import moe_layer
+
+    E, H, I = 4, 256, 256
+    L = moe_layer(seed=3, experts=E, top_k=1, hidden=H, intermediate=I, tokens=1, qtype=qtype, down_qtype=down, pack=False)
+    fn = expert_parallel(None, gate_type=qtype, up_type=qtype, down_type=down, hidden=H, intermediate=I).with_mode(2)
+    tabs = fn.prepare(*(L[n].reshape(E, -1) for n in ("gate", "up", "down")), device)
+    for per, thin in ((max(most, 1), most > 0), (most + 1, False)):
+        tokens = E * per if thin else E * (per - 1) + 1
+        x = torch.randn(tokens, H, device=device).to(torch.bfloat16)
+        ids = (torch.arange(tokens, device=device, dtype=torch.int32) % E)[:, None]
+        w = torch.ones(tokens, 1, device=device, dtype=torch.bfloat16)
+        names = kernels(lambda: fn(*tabs, x, ids, w))
+        for phase in ("moe_pf_gate_up_kernel<", "moe_pf_down_kernel<"):
+            name, = [k for k in names if phase in k]
+            assert (", 64>" in name, ", 128>" in name) == (thin, not thin), (per, name)

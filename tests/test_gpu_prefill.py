@@ -196,3 +196,21 @@ def test_thin_tiles_of_every_width(device, qtype, down, hidden, inter):
     L2 = dict(L, x=np.concatenate([L["x"]] * 2), weights=np.concatenate([L["weights"]] * 2))
     twice, _ = _run(L2, device, mode=2, ids=np.concatenate([ids] * 2))
     np.testing.assert_array_equal(twice, np.concatenate([got, got]))
+
+
+@pytest.mark.parametrize("qtype,down", [("Q4_K", "Q8_0"), ("Q6_K", "Q5_1"), ("Q5_K", "Q6_K"), ("Q8_0", "Q4_K"),
+                                        ("Q6_K", "Q5_K")])
+def test_thin_tiles_of_mixed_formats(device, qtype, down):
+    # tiles of 64 routes with one projection of a format that keeps two waves per
+    # SIMD, up to 36 routes per expert; the same tokens twice run in tiles of 128
+    counts = [1, 16, 33, 64, 65, 129] + [0] * 5
+    experts, tokens = len(counts), sum(counts)
+    assert tokens <= 36 * experts < 48 * experts < 2 * tokens
+    L = moe_layer(seed=tokens, experts=experts, top_k=1, hidden=512, intermediate=256, tokens=tokens, qtype=qtype,
+                  down_qtype=down, pack=False)
+    ids = np.random.default_rng(9).permutation(np.repeat(np.arange(experts), counts)).astype(np.int32)[:, None]
+    got, _ = _run(L, device, mode=2, ids=ids)
+    assert_moe_close(got, _oracle(L, ids=ids))
+    L2 = dict(L, x=np.concatenate([L["x"]] * 2), weights=np.concatenate([L["weights"]] * 2))
+    twice, _ = _run(L2, device, mode=2, ids=np.concatenate([ids] * 2))
+    np.testing.assert_array_equal(twice, np.concatenate([got, got]))
