@@ -804,13 +804,12 @@ __device__ __forceinline__ void dec_gate_up_item(uint8_t* smem, uint8_t* ring, i
 }
 
 // Items: the shared expert's (row group, pass of 16 tokens) first (sh.is > 0),
-// then its gate, one token each, then (row group, expert slot) with the row
-// group fastest.
-template <int FMT, bool kFullK>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-    moe_dec_gate_up_kernel(Proj gate, Proj up, DecRoute R, DecTables T, const uint16_t* __restrict__ x,
-                           int hidden, uint16_t* __restrict__ act, int inter, DecShared sh) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+// then its gate, one token each (kGate), then (row group, expert slot) with the
+// row group fastest.
+template <int FMT, bool kFullK, bool kGate>
+__device__ __forceinline__ void dec_gate_up(uint8_t* smem, const Proj& gate, const Proj& up, const DecRoute& R,
+                                            const DecTables& T, const uint16_t* x, int hidden, uint16_t* act, int inter,
+                                            const DecShared& sh) {
   const int wave = split_wave();
   const int wl = gu_wave_lds<FMT>(R.B * R.K, R.E);
   uint8_t* ring = smem + wave * wl;
@@ -829,10 +828,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
                                   sh.is);
     return;
   }
-  const int first = sh_items + sh.gate_of.tokens;
-  if (item < first) {
-    if (wave == 0) shared_gate_token(sh.gate_of, item - sh_items, threadIdx.x & 63);
-    return;
+  int first = sh_items;
+  if constexpr (kGate) {
+    first += sh.gate_of.tokens;
+    if (item < first) {
+      if (wave == 0) shared_gate_token(sh.gate_of, item - sh_items, threadIdx.x & 63);
+      return;
+    }
   }
   const int groups_i = (inter + 15) / 16;
   const int rg = (item - first) % groups_i, slot = (item - first) / groups_i;
@@ -840,6 +842,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
   if (!dec_route(R, slot, rg == 0 && wave == 0, T, ring, tok, sr)) return;
   dec_gate_up_item<FMT, kFullK>(smem, ring, wl, gate, up, sr.expert, rg, sr.t0, sr.cnt, tok, x, R.B, hidden, act,
                                 inter);
+}
+
+// The launch with the shared expert's gate is compiled apart: its items' scalars
+// cost the launch without one 1.6-3.4 % of the whole step in Q4_K and Q5_K layers
+// (64 experts, top-6, H 2048, I 1536, Q4_K, 8 tokens: 52.4 us without, 53.4 with;
+// 256 experts, top-8, Q5_K, 32 tokens: 105.5 and 108.8).
+template <int FMT, bool kFullK>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    moe_dec_gate_up_kernel(Proj gate, Proj up, DecRoute R, DecTables T, const uint16_t* __restrict__ x,
+                           int hidden, uint16_t* __restrict__ act, int inter, DecShared sh) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  dec_gate_up<FMT, kFullK, false>(smem, gate, up, R, T, x, hidden, act, inter, sh);
+}
+template <int FMT, bool kFullK>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+    moe_dec_gate_up_gated_kernel(Proj gate, Proj up, DecRoute R, DecTables T, const uint16_t* __restrict__ x,
+                                 int hidden, uint16_t* __restrict__ act, int inter, DecShared sh) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  dec_gate_up<FMT, kFullK, true>(smem, gate, up, R, T, x, hidden, act, inter, sh);
 }
 
 // One routed down item: row groups kDownRows*blk.. of slot ``slot``'s expert,
@@ -1110,9 +1131,10 @@ static int launch(const DecArgs& A, hipStream_t s) {
   constexpr int lds_dn = ring_bytes<FD>();
   static std::atomic<uint64_t> attr_done{0};
   once_per_device(attr_done, [] {  // the most any launch asks for
-    (void)hipFuncSetAttribute((const void*)moe_dec_gate_up_kernel<FG, kFullK>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              4 * gu_wave_lds<FG>(kDecMaxEntries, kMaxExperts));
+    for (const void* k : {(const void*)moe_dec_gate_up_kernel<FG, kFullK>,
+                          (const void*)moe_dec_gate_up_gated_kernel<FG, kFullK>})
+      (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                4 * gu_wave_lds<FG>(kDecMaxEntries, kMaxExperts));
     (void)hipFuncSetAttribute((const void*)moe_dec_down_kernel<FD, kFullK>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, 4 * ring_bytes<FD>());
   });
@@ -1126,7 +1148,9 @@ static int launch(const DecArgs& A, hipStream_t s) {
   // 64 entries that every wave repeats cheaply
   const int kb_i = (int)cdiv(A.I, kQK);
   const bool long_dn = kb_i % 2 == 0 && kb_i >= 4 && A.R.B * A.R.K <= 64;
-  const unsigned grid_gu = (unsigned)(items_gu + (A.S.is ? A.S.gate_of.tokens : 0));
+  const int gate_items = A.S.is ? A.S.gate_of.tokens : 0;
+  const auto gate_up = gate_items ? moe_dec_gate_up_gated_kernel<FG, kFullK> : moe_dec_gate_up_kernel<FG, kFullK>;
+  const unsigned grid_gu = (unsigned)(items_gu + gate_items);
   const int ns_gu = split_for(items_gu, false), ns_dn = split_for(items_dn, long_dn);
   // One launch for gate/up and down where the routes are spread thin (fewer
   // than 0.4 routes per expert on average: most active experts see one route,
@@ -1160,11 +1184,11 @@ static int launch(const DecArgs& A, hipStream_t s) {
   } else {
     if (A.gate_up_start && A.after_gate_up) {
       // the events take the kernel's own start and end timestamps
-      hipExtLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3(grid_gu), dim3(64 * ns_gu),
+      hipExtLaunchKernelGGL(gate_up, dim3(grid_gu), dim3(64 * ns_gu),
                             ns_gu * lds_gu, s, (hipEvent_t)A.gate_up_start, (hipEvent_t)A.after_gate_up, 0, A.gate,
                             A.up, A.R, A.T, A.x, A.H, A.act, A.I, A.S);
     } else {
-      hipLaunchKernelGGL((moe_dec_gate_up_kernel<FG, kFullK>), dim3(grid_gu), dim3(64 * ns_gu),
+      hipLaunchKernelGGL(gate_up, dim3(grid_gu), dim3(64 * ns_gu),
                          ns_gu * lds_gu, s, A.gate, A.up, A.R, A.T, A.x, A.H, A.act, A.I, A.S);
       if (A.after_gate_up) (void)hipEventRecord((hipEvent_t)A.after_gate_up, s);
     }

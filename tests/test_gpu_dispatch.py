@@ -65,3 +65,21 @@ def test_tile_width_by_format_and_routes_per_expert(device, qtype, down, most):
         for phase in ("moe_pf_gate_up_kernel<", "moe_pf_down_kernel<"):
             name, = [k for k in names if phase in k]
             assert (", 64>" in name, ", 128>" in name) == (thin, not thin), (per, name)
+
+
+def test_decode_gate_up_without_a_gate_runs_without_its_items(device):
+    from q6moe.experts import expert_parallel, pack_experts
+    from q6moe.synth import moe_layer
+
+    L = moe_layer(seed=4, experts=4, top_k=2, hidden=256, intermediate=256, tokens=3, shared_intermediate=256, pack=False)
+    fn = expert_parallel(None, gate_type="Q6_K", up_type="Q6_K", down_type="Q6_K", hidden=256, intermediate=256)
+    tabs = fn.prepare(*(L[n].reshape(4, -1) for n in ("gate", "up", "down")), device)
+    sh = {n: pack_experts(L["shared"][n].reshape(1, -1), "Q6_K", 256, 256, device) for n in ("gate", "up", "down")}
+    sh["intermediate"] = 256
+    x = torch.from_numpy(L["x"]).to(device).to(torch.bfloat16)
+    ids, w = torch.from_numpy(L["ids"]).to(device), torch.from_numpy(L["weights"]).to(device).to(torch.bfloat16)
+    router = torch.ones(256, device=device, dtype=torch.bfloat16)
+    scale = torch.ones(3, device=device, dtype=torch.bfloat16)
+    for shared, gated in ((None, False), (sh, False), (dict(sh, scale=scale), False), (dict(sh, router=router), True)):
+        call = lambda: fn.with_mode(1)(*tabs, x, ids, w, shared=shared)  # noqa: E731
+        assert launched(call, "moe_dec_gate_up_gated_kernel") == gated
