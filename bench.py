@@ -798,8 +798,8 @@ def measure_q4_shared(dev, with_cpu):
                                   zip(("pre", "gate_up", "down", "combine") if b <= 64 else
                                       ("shared", "routed_gate_up", "routed_down", "combine"), ph)},
                     "active_experts": active, "bytes_per_step": nbytes, "layer_copies": want_copies,
-                    # above 48 tokens the layer runs on the grouped kernels
-                    "roofline": roofline("q6moe::moe_dec_gate_up_kernel<1, true>" if b <= 48 else
+                    # from 56 tokens on the layer runs on the grouped kernels
+                    "roofline": roofline("q6moe::moe_dec_gate_up_kernel<1, true>" if b < 56 else
                                          "q6moe::moe_pf_gate_up_kernel<1, true, 128>", "hbm", gu_bytes, ph[1],
                                          work_unit="bytes_per_launch", tag=f"{b} token")})
         out["batches"][str(b)] = row
@@ -882,9 +882,9 @@ def measure_wide_layer(dev, with_cpu):
             layers.append(clone_tables(base))
         x, ids, w = xa[:b].contiguous(), ida[:b].contiguous(), wa[:b].contiguous()
         # the operator's default family (mode 0): the decode-step kernels, or
-        # the grouped ones once tokens x top-k x experts reaches 2^16
+        # the grouped ones once tokens x top-k x experts reaches 2^17 (of these counts)
         f = fn
-        family = "grouped" if b * WIDE_K * WIDE_E >= 1 << 16 else "decode"
+        family = "grouped" if b * WIDE_K * WIDE_E >= 1 << 17 else "decode"
         ws = torch.empty(f.workspace_bytes(b, WIDE_K, WIDE_E), dtype=torch.uint8, device=dev)
         o = torch.empty((b, WIDE_H), dtype=torch.bfloat16, device=dev)
 

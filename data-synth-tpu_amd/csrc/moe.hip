@@ -1430,24 +1430,57 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
   // large (tokens x top-k x experts >= 2^17) and no shared expert rides along:
   // every decode-step wave repeats the routing over all entries and experts,
   // and an expert's (and the shared expert's) weights are decoded again for
-  // every 16 of its tokens. Where the tiled kernels take the layer and its
-  // experts' row blocks alone fill the chip (experts x blocks >= 1024), the
-  // grouped kernels are faster from 2^16 on, from 2.5 routes per expert, and
-  // with a shared expert above 48 tokens. Measured (us, decode against grouped;
-  // even and skewed loads): 512-expert top-10 Q6_K/Q8_0 layer, 12 tokens 114 and
-  // 118, 97 and 105; 16 tokens 139 and 138, 123 and 119; 32 tokens 240 and 210,
-  // 197 and 171. 128-expert top-8 Q6_K layer, 32 tokens 107 and 104, 88 and 89;
-  // 40 tokens 111 and 107, 99 and 92; 64 tokens 124 and 112, 123 and 101; its
-  // Q5_K/Q8_0 form, 40 tokens 123 and 126, 113 and 109; 64 tokens 138 and 130,
-  // 136 and 116. 64-expert top-6 Q4_K layer with a shared expert, 40 tokens 133
-  // and 148, 132 and 125; 48 tokens 138 and 148, 145 and 127; 64 tokens 151 and
-  // 148, 180 and 135. The workspace bound keeps the choice the same for the
-  // entry point on the static scratch, and no call is refused for it.
-  const bool dec_auto = B <= 64 && (Is > 0 || B * K * E < (int64_t(1) << 17));
+  // every 16 of its tokens. The grouped kernels route once and decode a weight
+  // once per tile, but start up twice more and need enough items at a time:
+  // experts x row blocks >= 1024 of gate/up and, below 16 routes per expert, >= 512
+  // of down (1024 with a shared expert's own items beside them). There they come
+  // earlier:
+  //   many  from 2.5 routes per expert, with formats that keep three workgroups
+  //         per CU; with others from 48 tokens;
+  //   big   from 2^16 on and 20 tokens, from 1.5 routes per expert with one such
+  //         format, from 0.4 (below, the decode step is one launch) with two and
+  //         experts of 2^20 weights per projection;
+  // with a shared expert from 49 tokens (big) or 56 (many, or 2^17 and 0.4 routes
+  // per expert). Measured (us, decode against grouped; even and skewed loads):
+  //   many  128 experts top-8 (H 2048, I 768) Q6_K, 32 tokens 103 and 102, 87 and
+  //         88; 40 tokens 109 and 107, 95 and 91. 32 top-4 (2048, 2048) Q6_K, 20
+  //         tokens 75 and 75, 65 and 63. Q4_K: 64 top-6 (2048, 1536), 32 tokens 93
+  //         and 97, 85 and 86; 48 tokens 98 and 98, 95 and 91. 32 top-4 (4096,
+  //         2048), 40 tokens 120 and 124, 115 and 114; 48 tokens 120 and 120, 122
+  //         and 120. Q5_K/Q8_0 128 top-8, 40 tokens 116 and 123, 102 and 106; 48
+  //         tokens 122 and 124, 107 and 108.
+  //   big   512 top-10 (2560, 640) Q6_K/Q8_0, 13 tokens 120 and 120, 99 and 100; 23
+  //         tokens 182 and 164, 158 and 143. 512 top-8 (2048, 512) Q8_0, 20 tokens
+  //         97 and 103, 81 and 87; 26 tokens 123 and 123, 107 and 106. 256 top-16
+  //         (1024, 256) Q6_K/Q8_0, 16 tokens 38 and 42; 24 tokens 54 and 49, 43 and
+  //         43. Q4_K 256 top-8 (2048, 512), 32 tokens 82 and 91; 48 tokens 107 and
+  //         112. 1024 top-8 (2048, 768) Q6_K, 8 tokens 49 and 59.
+  //   down  experts x blocks of 128: 8 top-2 (4096, 14336) Q6_K, 10 tokens 210 and
+  //         238; 16 top-4 (2048, 4096), 16 tokens 74 and 89; 8 top-2 (2048, 8192)
+  //         Q5_K, 40 tokens 81 and 112; 64 tokens (16 routes) 137 and 119; the
+  //         first 348 and 267.
+  //   shared  64 top-6 (4096, 1024, shared 4096) Q4_K, 49 tokens 136 and 147, 136
+  //         and 132; 56 tokens 138 and 146, 138 and 129; 64 tokens 145 and 147, 179
+  //         and 133. 256 top-8 Q6_K/Q8_0 (768), 49 tokens 195 and 181, 159 and 142.
+  //         16 top-2 (4096, 4096, 2048) Q6_K, 56 tokens 151 and 165. 64 top-1 Q8_0,
+  //         49 tokens 47 and 62; 128 top-4 Q5_K/Q8_0, 64 tokens 110 and 114.
+  // The workspace bound keeps the choice the same for the entry point on the static
+  // scratch; no call is refused for it, and a workspace of the queried size never
+  // meets it first.
+  const int64_t n = B * K;
+  const bool dec_auto = B <= 64 && (Is > 0 || n * E < (int64_t(1) << 17));
   const auto group_few = [&] {
-    if (!rows32 || !pf_gate_up_supported(fmt, H, I) || !pf_down_supported(fmt_dn, H, I) || E * (I / 64) < 1024)
+    if (!rows32 || !pf_gate_up_supported(fmt, H, I) || !pf_down_supported(fmt_dn, H, I)) return false;
+    if (E * (I / 64) < 1024 || (n < 16 * E && E * (H / 128) < (Is ? 1024 : 512))) return false;
+    if (Is && (!sh_tiled_gu || !sh_tiled_dn)) return false;
+    const int dense = pf_thin_dense(fmt) + pf_thin_dense(fmt_dn);
+    const bool one_launch = 5 * n < 2 * E;  // launch_moe_decode's fused form
+    const bool many = 2 * n >= 5 * E;
+    const bool big = B >= 20 && n * E >= (1 << 16) &&
+                     (2 * n >= 3 * E ? dense >= 1 : dense == 2 && !one_launch && H * I >= (1 << 20));
+    if (Is ? !((B >= 49 && big) || (B >= 56 && (many || (n * E >= (1 << 17) && !one_launch))))
+           : !(big || (many && (dense == 2 || B >= 48))))
       return false;
-    if (Is ? B <= 48 || !sh_tiled_gu || !sh_tiled_dn : B * K * E < (1 << 16) && 2 * B * K < 5 * E) return false;
     const size_t need = ws_layout(B, K, E, H, I, Is, kPrefillTile, false).total;
     return need <= kStaticScratchBytes && need <= workspace_bytes;
   };

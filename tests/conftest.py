@@ -29,6 +29,24 @@ def device():
     return torch.device("cuda", 0)
 
 
+@pytest.fixture
+def kernels(device):
+    """``kernels(call)``: the names of this library's kernels that ``call`` launches, from a trace."""
+    import torch
+
+    def names(call):
+        call()
+        torch.cuda.synchronize()
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as trace:
+            call()
+            torch.cuda.synchronize()
+        found = [e.key for e in trace.key_averages() if "q6moe::" in e.key]
+        assert found, "the trace holds no kernel of this library"
+        return found
+
+    return names
+
+
 def pytest_runtest_setup(item):
     if "gpu" in item.keywords:
         print(f"\n[gpu-test] {item.nodeid}", flush=True)

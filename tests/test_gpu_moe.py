@@ -591,11 +591,12 @@ def test_shared_gate_of_every_path(device, tokens, mode):
 
 
 @pytest.mark.parametrize("tokens,experts,top_k,shared,grouped", [
-    (39, 128, 8, 0, False), (40, 128, 8, 0, True),      # 2.5 routes per expert
-    (15, 512, 8, 0, False), (16, 512, 8, 0, True),      # tokens x top-k x experts of 2^16
+    (47, 128, 8, 0, False), (48, 128, 8, 0, True),      # 48 tokens at 2.5 routes per expert and more
+    (31, 512, 8, 0, False), (32, 512, 8, 0, True),      # tokens x top-k x experts of 2^17
     (64, 64, 8, 0, False),                              # experts x row blocks below 1024
-    (48, 128, 4, 256, False), (49, 128, 4, 256, True),  # with a shared expert above 48 tokens
-    (64, 128, 4, 96, False),                            # whose shape the tiled kernels do not take
+    (55, 128, 8, 256, False), (56, 128, 8, 256, True),  # with a shared expert from 56 tokens
+    (64, 128, 4, 256, False),                           # and 2.5 routes per expert
+    (64, 128, 8, 96, False),                            # whose shape the tiled kernels do not take
 ])
 def test_default_family_by_size(device, tokens, experts, top_k, shared, grouped):
     # Both families run every one of these calls; the default one gives the bits

@@ -144,23 +144,24 @@ def test_noalloc_call_replays_in_a_captured_graph(device, case):
     del keep
 
 
-def test_noalloc_keeps_the_decode_kernels_where_the_grouped_ones_need_more_scratch(device):
-    # 32 tokens, top-32 of 40 experts: the default rule prefers the grouped
+def test_noalloc_keeps_the_decode_kernels_where_the_grouped_ones_need_more_scratch(device, kernels):
+    # 32 tokens, top-32 of 64 experts: the default rule prefers the grouped
     # kernels, whose regions exceed the scratch at this width; the decode-step ones
-    # fit, and both entry points run them.
-    E, H, I, B, K = 40, 128, 11264, 32, 32
-    rng = np.random.default_rng(5)
+    # fit, and both entry points run them. At top-16 both families fit.
+    E, H, I, B = 64, 1024, 11264, 32
 
     def table(rows, width):
-        raw = rng.integers(0, 256, (E, rows, width // 32, 34), dtype=np.uint8)
-        raw[..., :2] = np.array([0.0005], np.float16).view(np.uint8)
+        raw = torch.randint(0, 256, (E, rows, width // 32, 34), dtype=torch.uint8, device=device)
+        raw[..., :2] = torch.tensor([0.0005], dtype=torch.float16, device=device).view(torch.uint8)
         return raw.reshape(E, -1)
 
     fn = expert_parallel(None, gate_type="Q8_0", up_type="Q8_0", down_type="Q8_0", hidden=H, intermediate=I)
     tabs = fn.prepare(table(I, H), table(I, H), table(H, I), device)
     x = torch.randn(B, H, device=device).to(torch.bfloat16)
-    ids = torch.rand(B, E, device=device).topk(K).indices.to(torch.int32)
-    w = torch.rand(B, K, device=device).to(torch.bfloat16)
-    assert fn.workspace_bytes(B, K, E) > SCRATCH_BYTES
-    want, got = _both(fn, tabs, device, x, ids, w, mode=0)
-    np.testing.assert_array_equal(got, want)
+    for K, grouped in ((32, False), (16, True)):
+        ids = torch.rand(B, E, device=device).topk(K).indices.to(torch.int32)
+        w = torch.rand(B, K, device=device).to(torch.bfloat16)
+        assert (fn.workspace_bytes(B, K, E) > SCRATCH_BYTES) != grouped
+        assert any("moe_pf_gate_up_kernel" in k for k in kernels(lambda: fn(*tabs, x, ids, w))) == grouped
+        want, got = _both(fn, tabs, device, x, ids, w, mode=0)
+        np.testing.assert_array_equal(got, want)
