@@ -295,13 +295,15 @@ extern "C" int q6moe_q6_matmul(const uint16_t* x, int64_t m, int64_t k, int64_t 
   const int xvec = (ldx % 8 == 0) && aligned(x, 16);
   const int ybf16 = y_dtype == Q6MOE_BF16;
   hipStream_t s = (hipStream_t)stream;
-  // The tiled kernel from 64 tokens on, and above 16 for up to three K blocks:
-  // its K blocks pass one after another in each set (~1.2 us each with few
-  // workgroups), the skinny kernel's all at once. 1280 x 2560: 48 tokens 11.0 us
-  // skinny and 12.7 tiled, 64 tokens 13.0 and 12.8, 777 tokens 49.0 and 20.3;
-  // 1000 x 520: 17 tokens 8.6 and 5.9; 2048 x 1024: 17 tokens 5.6 and 6.9. It
-  // needs whole 16-byte groups of x and 32-bit offsets into it.
-  const bool tiled = (m >= 64 || (m > 16 && kb <= 3)) && xvec && k % 8 == 0 && (m + 63) * ldx * 2 < (1ll << 31);
+  // The tiled kernel from 64 tokens on, and above 16 for up to five 128-wide halves
+  // of K: its halves pass one after another in each set (~0.6 us each with few
+  // workgroups), the skinny kernel's blocks all at once. Skinny and tiled (us),
+  // 17 and 48 tokens: 1280 x 256 6.4 and 4.7, 6.8 and 5.0; x 512 5.5 and 5.2, 5.9
+  // and 5.5; x 640 7.4 and 6.3, 8.6 and 6.5; x 736 6.6 and 7.0, 7.5 and 7.2; x 768
+  // 5.5 and 6.9, 6.5 and 7.2, with 63 tokens 7.2 and 7.3; 1280 x 2560, 48 tokens 11.0
+  // and 12.7, 64 tokens 13.0 and 12.8, 777 tokens 49.0 and 20.3. It needs whole
+  // 16-byte groups of x and 32-bit offsets into it.
+  const bool tiled = (m >= 64 || (m > 16 && k <= 640)) && xvec && k % 8 == 0 && (m + 63) * ldx * 2 < (1ll << 31);
   if (tiled) {
     // four K sets where the workgroups leave CUs idle (1280 x 2560, 256 tokens:
     // 13.0 us against 13.9 with two; 777 tokens, 260 workgroups: 26.4 against 20.3)

@@ -119,3 +119,18 @@ def test_default_family_by_size_and_format(device, kernels, qtype, down, experts
     names = kernels(lambda: fn(*tabs, x, ids, w, shared=sh))
     assert any("moe_pf_gate_up_kernel" in k for k in names) == grouped
     assert any("moe_dec_" in k for k in names) != grouped
+
+
+@pytest.mark.parametrize("inputs,tokens,tiled", [
+    (640, 16, False), (640, 17, True), (648, 17, False), (768, 63, False), (768, 64, True), (2560, 63, False),
+    (2560, 64, True)])
+def test_projection_kernel_by_size(device, kernels, inputs, tokens, tiled):
+    from oracle import packed_q6
+    from q6moe import pack_q6
+    from q6moe.kernel import q6_matmul
+
+    p = pack_q6(packed_q6.fixture(64, inputs), inputs)
+    data, scales = torch.from_numpy(p.data).to(device), torch.from_numpy(p.scales).to(device)
+    x = torch.randn(tokens, inputs, device=device).to(torch.bfloat16)
+    names = kernels(lambda: q6_matmul(x, data, scales, output_features=64))
+    assert any("q6_tile_kernel" in k for k in names) == tiled

@@ -246,10 +246,10 @@ def test_dequantize_rows_hip_staged_and_fallback_paths(device, qtype):
 
 
 @pytest.mark.parametrize("batch,outputs,inputs", [
-    (17, 130, 520), (17, 3, 8), (40, 64, 768), (64, 64, 256), (65, 67, 1544), (127, 320, 2560), (128, 65, 1408),
+    (17, 130, 520), (17, 3, 8), (40, 64, 640), (64, 64, 256), (65, 67, 1544), (127, 320, 2560), (128, 65, 1408),
     (200, 96, 3080), (64, 16448, 256)])
 def test_tiled_projection(device, batch, outputs, inputs):
-    # 64-token tiles from 64 tokens on (17 with up to three K blocks): one token
+    # 64-token tiles from 64 tokens on (17 with up to 640 inputs): one token
     # past a tile, rows past the matrix, K ending inside a 128-wide half, K sets of
     # unequal (or no) blocks, two and four sets. x is a view of wider rows whose
     # padding must not enter.
