@@ -1293,8 +1293,6 @@ extern "C" int q6moe_moe_unpack(const uint8_t* table, int qtype, int64_t experts
                     width <= (1 << 24) && (!block32_qtype(qtype) || width % 32 == 0),
                 "moe_unpack: bad shape");
   Q6MOE_REQUIRE(path >= 0 && path <= 2, "moe_unpack: path must be 0 (generic), 1 (decode) or 2 (prefill)");
-  Q6MOE_REQUIRE(path != 2 || pf_unpack_supported(fmt_of(qtype)),
-                "moe_unpack: the prefill path decodes Q6_K, Q8_0, Q5_1 and Q4_K");
   const int64_t need = unit_table_bytes(qtype, rows, width);
   Q6MOE_REQUIRE(aligned(table, 16) && (experts == 1 || (stride >= need && stride % 16 == 0)),
                 "moe_unpack: table must be 16-byte aligned with a stride covering one expert");

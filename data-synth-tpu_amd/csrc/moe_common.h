@@ -229,7 +229,6 @@ int launch_moe_decode(int fmt_gu, int fmt_dn, const DecArgs& A, hipStream_t s);
 // Unit-decode probes (q6moe_moe_unpack): the decode kernels' LDS-staged path
 // and the prefill kernels' whole-block register path, for the bit-exact tests.
 int launch_dec_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStream_t s);
-bool pf_unpack_supported(int fmt);
 int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStream_t s);
 
 // Prefill grouped GEMM, tiled on the matrix cores: gate/up (every format but

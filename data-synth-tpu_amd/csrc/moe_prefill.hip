@@ -51,8 +51,6 @@ int launch_moe_prefill_down(int fmt, const Proj& d, const MoeWs& ws, int mtile, 
   return Q6MOE_OK;
 }
 
-bool pf_unpack_supported(int fmt) { return fmt == FMT_Q6 || fmt == FMT_Q8 || fmt == FMT_Q51 || fmt == FMT_Q4K; }
-
 int launch_pf_unpack(int fmt, const Proj& p, int experts, uint16_t* out, hipStream_t s) {
   dispatch_format(fmt, [&](auto fc) { pf_unpack<decltype(fc)::value>(p, experts, out, s); });
   return Q6MOE_OK;

@@ -138,7 +138,7 @@ int q6moe_moe_pack(const uint8_t* raw, int qtype, int64_t experts, int64_t rows,
  * code is 32 decodes to +0 whatever the sign of d*sc). ``path`` picks the
  * decoder the MoE kernels use: 0 the generic kernels' register decode, 1 the
  * decode-step kernels' LDS-staged decode, 2 the prefill kernels' whole-block
- * decode (Q6_K only). No counterpart call in the reference: it is the
+ * decode. No counterpart call in the reference: it is the
  * unit-major analogue of q6moe_q6_decode, for tests of the decoders.
  */
 int q6moe_moe_unpack(const uint8_t* table, int qtype, int64_t experts, int64_t rows, int64_t width,
