@@ -61,11 +61,6 @@ class ExpertTable:
     def experts(self):
         return self.data.shape[0]
 
-    def c_table(self):
-        t = _lib.Table()
-        self.fill(t)
-        return t
-
     def fill(self, t):
         """Writes this table into the C structure ``t`` (zeroed, as ctypes makes it)."""
         t.qtype = _lib.QTYPE_CODES[self.qtype]
