@@ -222,14 +222,16 @@ struct Block<FMT_Q4K> : NoFold {
 // Q5_K, with Q4_K's lane map (in K half h the lane decodes sub-block s = 4h + jA,
 // fragment f its positions 8f + [0, 8)): nibbles in chunks 3 + 2c and 4 + 2c of
 // the unit (c = 2h + jA/2), bit s of the 32 high-bit bytes (chunks 1, 2) as bit
-// 4. ``pin`` keeps the lane's two bits per high-bit byte in two words (28
-// registers per unit while loading, 22 from then on): bit i of the low (high)
-// nibble of byte b of word p is the fifth bit of position 16p + 4i + b of K
-// half 0 (1). Nibble and fifth bit meet as FP16 subnormals (sub_frag): the
+// 4. ``fold`` leaves the lane's two bits per high-bit byte in two words: bit i of
+// the low (high) nibble of byte b of word p is the fifth bit of position 16p + 4i
+// + b of K half 0 (1). Nibble and fifth bit meet as FP16 subnormals (sub_frag): the
 // nibbles of bytes 0 and 2 of a code word at bits 0-3 (4-7 for an odd
 // sub-block) of its halves, the fifth bits rotated to bit 4 (8); bytes 1 and 3
 // the same after a shift by 8. w = fma(q, d*sc, -dmin*m), one rounding, RNE to
-// BF16 (gguf_quant.py:115-157).
+// BF16 (gguf_quant.py:115-157). With the most registers per unit (28), the
+// 128-route kernels spill 7-10 where a tile holds 113-128 routes; the 64-route ones
+// take 208. Pinning only the folded words after the fold spills 8-12 and is no
+// faster (128-expert top-8 layer, 2048 tokens 309.5 us as here, 311.3 so).
 template <>
 struct Block<FMT_Q5K> {
   static constexpr int kLoads = 7;
