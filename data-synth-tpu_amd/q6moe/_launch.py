@@ -10,19 +10,18 @@ import torch
 
 from . import _lib
 
-_current_device = torch._C._cuda_getDevice
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
 def run(what, fn, device, *args):
     """``fn(*args, stream)`` with ``device`` (a GPU tensor's, so with an index) current; raises on an error code."""
     if device.type != "cuda":
         raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
-    if index == _current_device():
-        rc = fn(*args, _raw_stream(index))
+    # looked up per call: a torch built without a GPU backend lacks both names, and
+    # still imports the package
+    raw_stream = torch._C._cuda_getCurrentRawStream
+    if index == torch._C._cuda_getDevice():
+        rc = fn(*args, raw_stream(index))
     else:
         with torch.cuda.device(index):
-            rc = fn(*args, _raw_stream(index))
+            rc = fn(*args, raw_stream(index))
     if rc:
         _lib.check(rc, what)

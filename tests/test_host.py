@@ -2,7 +2,10 @@
 C-ABI library's exported symbols."""
 
 import ctypes
+import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -217,3 +220,17 @@ def test_attention_workspace_serves_every_smaller_call():
             sizes = [int(size(b, kvh * r, kvh, pps, 64)) for b in range(1, 20)]
             assert sizes == [need(b, kvh * r, kvh, pps * 64) for b in range(1, 20)]
             assert sizes == sorted(sizes)
+
+
+def test_package_imports_on_a_torch_without_a_gpu_backend():
+    code = ("import sys, torch\n"
+            "for n in ('_cuda_getDevice', '_cuda_getCurrentRawStream'):\n"
+            "    if hasattr(torch._C, n): delattr(torch._C, n)\n"
+            "import q6moe, q6moe._launch, q6moe.experts, q6moe.attention_cache, q6moe.compute\n"
+            "try:\n"
+            "    q6moe._launch.run('x', None, torch.device('cpu'))\n"
+            "except ValueError as e:\n"
+            "    print(e)\n")
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
+                         env=dict(os.environ, PYTHONPATH=str(ROOT / "data-synth-tpu_amd")))
+    assert "Expected a cuda device" in out.stdout, out.stderr[-500:]
