@@ -211,7 +211,7 @@ def read_paged(pool, scales, page_table, *, page_size, kv_heads, head_dim, group
     return out
 
 
-@lru_cache(maxsize=256)
+@lru_cache(maxsize=256, typed=True)
 def _attn_workspace_bytes(batch, hq, kv_heads, pps, page_size):
     return int(_lib.load().q6moe_attn_workspace_size(batch, hq, kv_heads, pps, page_size))
 

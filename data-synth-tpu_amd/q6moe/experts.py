@@ -233,7 +233,7 @@ def _check_workspace(workspace, need, device):
     return workspace
 
 
-@lru_cache(maxsize=256)
+@lru_cache(maxsize=256, typed=True)  # a value of another type is converted, or refused, as on a first call
 def _workspace_bytes(tokens, top_k, experts, hidden, intermediate, shared_intermediate):
     return int(_lib.load().q6moe_moe_workspace_size(tokens, top_k, experts, hidden, intermediate,
                                                     shared_intermediate))

@@ -234,3 +234,14 @@ def test_package_imports_on_a_torch_without_a_gpu_backend():
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120,
                          env=dict(os.environ, PYTHONPATH=str(ROOT / "data-synth-tpu_amd")))
     assert "Expected a cuda device" in out.stdout, out.stderr[-500:]
+
+
+def test_workspace_sizes_refuse_the_same_arguments_on_every_call():
+    # the sizes are kept by argument: 8.0 equals 8 and must not find its entry
+    from q6moe.experts import expert_parallel
+
+    fn = expert_parallel(None, gate_type="Q6_K", up_type="Q6_K", down_type="Q6_K", hidden=256, intermediate=256)
+    for _ in range(2):
+        assert fn.workspace_bytes(8, 2, 4) > 0
+        with pytest.raises(ctypes.ArgumentError):
+            fn.workspace_bytes(8.0, 2, 4)
