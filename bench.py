@@ -24,9 +24,11 @@ baseline leg, the CPU oracle's values within tolerance: max relative error
 1e-2 for the MoE, rtol 2e-5 / atol 2e-4 for the projection, bit-exact for the
 KV gather); a failure prints an error line and exits with status 1.
 
-Besides the headline line's ``roofline`` (moe_dec_gate_up_kernel, HIP events
-recorded between the launches on their stream) and ``cpu_baseline``, the
-``configs`` block carries, per workload: throughput with tokens/s, the median,
+The printed line holds the headline workload's block whole, with its
+``roofline`` (moe_dec_gate_up_kernel, HIP events recorded between the launches
+on their stream) and ``cpu_baseline``, and each other workload's throughput and
+time; ``--details FILE`` writes the whole record, whose ``configs`` block
+carries, per workload: throughput with tokens/s, the median,
 min and max over seeded interleaved repetitions of every method
 (kaggle/packed_q6/benchmark.py:127-154), the dominant kernel's roofline, the
 HBM traffic per launch from the committed rocprofv3 counter summaries
@@ -138,6 +140,35 @@ def roofline(kernel, bound, work, avg_us, *, work_unit, tag=None):
     return {"kernel": kernel, "bound": bound, "achieved": round(achieved, 1), "peak": peak, "unit": unit,
             "frac": round(achieved / peak, 4), "traffic": traffic, "traffic_source": source,
             work_unit: int(work), "avg_launch_us": round(float(avg_us), 3)}
+
+
+# What the printed line keeps of each workload's block.
+LINE_KEYS = ("value", "unit", "us_per_step", "us_per_call", "GBps", "tokens_per_s", "mfma_fraction", "hbm_fraction")
+LINE_SKIPS = ("cpu_baseline", "check", "roofline", "down_roofline")
+
+
+def summary(block):
+    """The LINE_KEYS of a workload's block, and of the blocks inside it that have any."""
+    if isinstance(block, list):
+        return []
+    kept = {k: v for k, v in block.items() if k in LINE_KEYS and isinstance(v, (int, float, str))}
+    for k, v in block.items():
+        if isinstance(v, dict) and k not in LINE_SKIPS and (inner := summary(v)):
+            kept[k] = inner
+    return kept
+
+
+def headline(result):
+    """The printed line: the headline workload whole, the others' summaries. The
+    whole record is several times as long, more than a log's tail holds of one line."""
+    line = {k: v for k, v in result.items() if k not in ("configs", "extras", "prefill", "step_us",
+                                                         "baselines_us_per_step")}
+    for k in ("configs", "extras"):
+        if k in result:
+            line[k] = {n: s for n, b in result[k].items() if (s := summary(b))}
+    if "prefill" in line.get("configs", {}):
+        line["prefill"] = line["configs"].pop("prefill")
+    return line
 
 
 def check_close(name, got, want, *, rel=1e-2, exact_frac=0.9):
@@ -718,7 +749,7 @@ def measure_prefill(dev, steps, warmup, with_cpu, down_qtype="Q6_K"):
         "phases_us": {k: round(float(v), 1) for k, v in zip(("route", "gate_up", "down", "combine"), ph)},
         "roofline": roofline("q6moe::moe_pf_gate_up_kernel<0, false, 128>", "mfma", PREFILL_FLOPS * 2 / 3, ph[1],
                              work_unit="flops_per_launch", tag="4096 tokens"),
-        "down_roofline": roofline(f"q6moe::moe_pf_down_kernel<{PF_FORMAT_ID[down_qtype]}>", "mfma",
+        "down_roofline": roofline(f"q6moe::moe_pf_down_kernel<{PF_FORMAT_ID[down_qtype]}, false, 128>", "mfma",
                                   PREFILL_FLOPS / 3, ph[2], work_unit="flops_per_launch", tag="4096 tokens"),
     })
     return res
@@ -789,18 +820,16 @@ def measure_q4_shared(dev, with_cpu):
         us = t["fused"]["median"]
         ph = phase_means(call, 50)
         gu_bytes = active * 2 * proj_bytes + b * H4 * 2 + routes * I4 * 2  # gate+up, x, SwiGLU rows
-        if b <= 64:  # the shared expert's gate/up run in the same launch
-            gu_bytes += 2 * IS * (H4 // 256) * 144 + b * IS * 2
+        gu_bytes += 2 * IS * (H4 // 256) * 144 + b * IS * 2  # the shared expert's, in the same launch
+        grouped = b >= 56  # the default family of this layer
         row.update({"us_per_step": round(us, 2), "GBps": round(nbytes / (us * 1e-6) / 1e9, 1),
                     "tokens_per_s": round(b / (us * 1e-6), 1),
                     "hbm_fraction": round(nbytes / (us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4), "step_us": t["fused"],
                     "phases_us": {k: round(float(v), 2) for k, v in
-                                  zip(("pre", "gate_up", "down", "combine") if b <= 64 else
-                                      ("shared", "routed_gate_up", "routed_down", "combine"), ph)},
+                                  zip(("route" if grouped else "pre", "gate_up", "down", "combine"), ph)},
                     "active_experts": active, "bytes_per_step": nbytes, "layer_copies": want_copies,
-                    # from 56 tokens on the layer runs on the grouped kernels
-                    "roofline": roofline("q6moe::moe_dec_gate_up_kernel<1, true>" if b < 56 else
-                                         "q6moe::moe_pf_gate_up_kernel<1, true, 128>", "hbm", gu_bytes, ph[1],
+                    "roofline": roofline("q6moe::moe_pf_gate_up_kernel<1, true, 128>" if grouped else
+                                         "q6moe::moe_dec_gate_up_kernel<1, true>", "hbm", gu_bytes, ph[1],
                                          work_unit="bytes_per_launch", tag=f"{b} token")})
         out["batches"][str(b)] = row
     return out
@@ -1072,6 +1101,7 @@ def main():
     ap.add_argument("--calib-copy-mb", type=int, default=0,
                     help="first copy a buffer of this many MiB device-to-device 5 times (a known-size "
                          "kernel for scaling hardware byte counters)")
+    ap.add_argument("--details", metavar="FILE", help="write the whole record (every workload's block) to FILE")
     ap.add_argument("--watchdog", type=int, default=900,
                     help="run the measurement in a child process and kill it after this many seconds "
                          "(exit status 124), as the reference harness supervises its worker; 0 runs it in "
@@ -1274,10 +1304,10 @@ def run(args):
                                         "kv_gather": measure_kv_harness(dev)}
         log("timing the compute policy gate (bf16 against int8_q8) ...")
         configs["compute_policy"] = measure_policy(dev)
-    if "prefill" in configs:
-        result["prefill"] = configs["prefill"]
     result["configs"] = configs
-    print(json.dumps(result), flush=True)
+    if args.details:
+        Path(args.details).write_text(json.dumps(result, indent=1) + "\n")
+    print(json.dumps(headline(result)), flush=True)
     return 0
 
 

@@ -66,8 +66,9 @@ def test_traffic_comes_from_the_committed_counter_summary():
     assert 120e6 < t < 140e6
     # per-workload rows of one kernel are told apart by their note
     t1, _ = bench.traffic_of("q6moe::moe_dec_gate_up_kernel<1, true>", tag="1 token")
-    t64, _ = bench.traffic_of("q6moe::moe_dec_gate_up_kernel<1, true>", tag="64 token")
-    assert t1 is not None and t64 is not None and t64 > 4 * t1
+    t8, _ = bench.traffic_of("q6moe::moe_dec_gate_up_kernel<1, true>", tag="8 token")
+    t64, _ = bench.traffic_of("q6moe::moe_pf_gate_up_kernel<1, true, 128>", tag="64 token")
+    assert t1 is not None and t8 > 3 * t1 and t64 > 4 * t1
 
 
 def test_stats_of_repetitions():
@@ -81,3 +82,21 @@ def test_more_than_one_gpu_is_refused_without_touching_a_gpu():
     assert p.returncode == 2
     assert "one GPU" in p.stderr
     assert p.stdout == ""
+
+
+def test_the_printed_line_keeps_the_contract_and_stays_short():
+    import json
+
+    block = {"value": 1.5, "unit": "GB/s", "us_per_step": 3.25, "tokens_per_s": 1e6, "workload": "w" * 80,
+             "step_us": {"median": 1.0, "min": 1.0, "max": 1.0, "mean": 1.0, "n": 7}, "check": {"value": 1},
+             "cpu_baseline": {"value": 2.0, "sample": "s" * 200}, "roofline": {"kernel": "k" * 50, "unit": "GB/s"}}
+    result = {"metric": bench.METRIC, "value": 1.0, "unit": "GB/s", "n_gpus": 1, "steps": 20, "warmup": 5,
+              "ms_per_step": 0.05, "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "bf16",
+              "data": "synthetic", "config": {"experts": 128}, "roofline": block["roofline"],
+              "configs": {f"c{i}": dict(block, batches={str(b): block for b in (1, 8, 64)}) for i in range(8)},
+              "extras": {"copy": block, "many": [block] * 30}}
+    line = bench.headline(result)
+    assert all(line[k] == result[k] for k in result if k not in ("configs", "extras"))
+    assert line["configs"]["c3"]["batches"]["8"] == {"value": 1.5, "unit": "GB/s", "us_per_step": 3.25,
+                                                     "tokens_per_s": 1e6}
+    assert len(json.dumps(line)) < 6000 < len(json.dumps(result))
