@@ -165,8 +165,10 @@ def test_one_workspace_serves_every_smaller_call(device, kvh, r, pps):
     ws = torch.empty(int(size(most, kvh * r, kvh, pps, page_size)), dtype=torch.uint8, device=device)
     for batch in range(most, 0, -1):
         lens = torch.tensor(lengths[:batch], dtype=torch.int32, device=device)
-        call = lambda **kw: paged_decode_attention(qt[:batch], *args, tt[:batch], lens, page_size=page_size,  # noqa: E731
-                                                   kv_heads=kvh, **kw)
+
+        def call(**kw):
+            return paged_decode_attention(qt[:batch], *args, tt[:batch], lens, page_size=page_size, kv_heads=kvh, **kw)
+
         got = call(workspace=ws)
         assert torch.equal(got, call())
         exact = int(size(batch, kvh * r, kvh, pps, page_size))
@@ -174,8 +176,8 @@ def test_one_workspace_serves_every_smaller_call(device, kvh, r, pps):
         with pytest.raises(ValueError, match="workspace"):
             call(workspace=ws[:exact - 1])
         if batch in (1, 3):
-            want = _want(pools, scales, table[:batch], qt[:batch].float().cpu().numpy(), lengths[:batch], page_size, kvh)
-            _check(got.float().cpu().numpy(), want)
+            qv = qt[:batch].float().cpu().numpy()
+            _check(got.float().cpu().numpy(), _want(pools, scales, table[:batch], qv, lengths[:batch], page_size, kvh))
 
 
 @pytest.mark.parametrize("pps,page_size", [(1, 64), (3, 64), (8, 64), (9, 64), (11, 64), (12, 64), (13, 128)])
