@@ -312,7 +312,9 @@ __global__ void __launch_bounds__(kPvThreads) __attribute__((amdgpu_waves_per_eu
         // exp(score - max) / sum, the correctly rounded quotient (Markstein, IBM
         // J. Res. Dev. 34, 1990): the rounded reciprocal's product and one
         // correction by the exact FMA residual, three instructions for each of
-        // the head's tokens
+        // the head's tokens. (Below 2^-103 the residual underflows and the last bit
+        // of the quotient may differ: nothing beside the largest probability, at
+        // least 1 / tokens, shows it.)
         const float e = expf(bf16_to_float(sc[i][h]) - sm[h]);
         q = e * si[h];
         q = bf16_round(__builtin_fmaf(__builtin_fmaf(-q, sl[h], e), si[h], q));

@@ -6,9 +6,11 @@
 // BF16: the order of moe_w8_kernel's waves (one block each up to 2048 inputs), so
 // that the number of tokens does not show, and no chain is longer than its own.
 //
-// Bound by the vector ALU: each partial product takes a conversion, a multiply
-// by the token's scale and a fused multiply-add by the row's (v_fma_mix_f32,
-// the FP16 scale as it lies in the unit), 12 instructions per MFMA. One
+// Bound by the vector ALU first: each partial product takes a conversion, a
+// multiply by the token's scale and a fused multiply-add by the row's
+// (v_fma_mix_f32, the FP16 scale as it lies in the unit), 12 instructions per MFMA,
+// which issue in 66 % (gate/up) and 57 % (down) of a SIMD's cycles at the step
+// below; a wave waits 27 % of its time, for a K block's weights and DMA. One
 // workgroup of 4 waves takes up to 64 routes of a tile against 64 rows of gate
 // and up, or 128 rows of down; each wave owns 2 units (16 weight rows x one
 // 256-wide K block) per K block, whose codes and scales it loads straight into

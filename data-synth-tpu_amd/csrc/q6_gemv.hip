@@ -101,9 +101,12 @@ __global__ void __launch_bounds__(512) q6_skinny_kernel(const uint16_t* __restri
 // columns past K and rows past m arrive as zeros (their lanes address past the
 // buffer's end; m > 16, so that the wave-uniform part of an address, at most one
 // row and 12 rows on, stays inside). The sets' sums meet in LDS in set order.
-// Bound by the decode: 232 vector instructions per unit and 64 tokens, at up to
-// four waves per SIMD (128 registers). 777 tokens, 2560 -> 1280: 49.0 -> 20.3
-// us (251 TFLOP/s); 1024 tokens, 4096 -> 4096: 294 -> 67.6 us (508 TFLOP/s).
+// Bound by waiting, with about one workgroup per CU: 777 tokens, 2560 -> 1280 (260
+// workgroups), the vector ALU issues in 38 % of a SIMD's cycles (232 instructions
+// of decode per unit and 64 tokens), the matrix cores work in 15 %, and a wave
+// spends 49 % of its time waiting, mostly for a half's DMA and the next weights,
+// issued one step before. 49.0 -> 20.3 us (251 TFLOP/s); 1024 tokens, 4096 -> 4096:
+// 294 -> 67.6 us (508 TFLOP/s).
 // ---------------------------------------------------------------------------
 namespace pj {
 

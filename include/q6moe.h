@@ -180,9 +180,13 @@ typedef struct q6moe_moe_args {
   void* workspace;             /* >= q6moe_moe_workspace_size(...) bytes, 256-byte aligned */
   size_t workspace_bytes;
   /* kernel family: 0 the decode-step kernels up to 64 tokens while the routing is small and
-     the experts see few routes each, else the grouped ones; 1 the decode-step kernels (B <= 256, B*top_k <= 1024, E <= 1024 and
+     the experts see few routes each, else the grouped ones (the families add in different
+     orders; a workspace smaller than q6moe_moe_workspace_size gives, where a call takes it
+     at all, can hold the decode-step kernels' regions only, and then runs those); 1 the
+     decode-step kernels (B <= 256, B*top_k <= 1024, E <= 1024 and
      B*top_k*max(H, I, Is) < 2^30, else Q6MOE_ERR_INVALID); 2 the grouped-GEMM (prefill)
-     kernels, tiled on the matrix cores for Q6_K with H and I multiples of 256 */
+     kernels, tiled on the matrix cores for gate/up with H a multiple of 128 and I of 64, for
+     down with I and H multiples of 128, in every table format */
   int mode;
   /* optional profiling: NULL, or Q6MOE_MOE_EVENTS hipEvent_t handles recorded on ``stream``
      before routing, after routing, after gate/up, after down, after the combine; on the
