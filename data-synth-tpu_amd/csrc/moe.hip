@@ -181,7 +181,9 @@ __device__ __forceinline__ void route_merge(const int* s_ids, float* s_w, int* c
 }
 
 // The workgroups from ``first`` on compute the shared expert's gate, one token
-// per wave. Returns whether this workgroup is one of them.
+// per wave. Returns whether this workgroup is one of them. The launches with a
+// gate are kernels of their own: its code made the one-launch routing without
+// one slower (1 token, 128 experts: 4.4 -> 5.2 us).
 __device__ __forceinline__ bool gate_block(const SharedGate& g, int first) {
   if ((int)blockIdx.x < first) return false;
   const int b = ((int)blockIdx.x - first) * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -193,11 +195,9 @@ __device__ __forceinline__ bool gate_block(const SharedGate& g, int first) {
 // token): merged BF16 weight of each first occurrence of an id in a token
 // (experts.py:66-73; 0 for repeats and out-of-range ids) and the chunk's
 // route count per expert.
-__global__ void __launch_bounds__(kChunk)
-    moe_route_count_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K,
-                           int E, int nchunks, MoeWs ws, int* __restrict__ chunk_cnt, SharedGate gate) {
+__device__ __forceinline__ void route_count(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B,
+                                            int K, int E, const MoeWs& ws, int* __restrict__ chunk_cnt) {
   extern __shared__ int sm[];
-  if (gate_block(gate, nchunks)) return;
   int* s_ids = sm;                                            // [kChunk * K]
   float* s_w = reinterpret_cast<float*>(sm + kChunk * K);     // [kChunk * K] weights, then merged weights
   __shared__ int cnt[kMaxExperts];
@@ -212,6 +212,17 @@ __global__ void __launch_bounds__(kChunk)
   __syncthreads();
   for (int i = tid; i < nb * K; i += kChunk) ws.ent_r[e0 + i] = s_w[i];
   for (int e = tid; e < E; e += kChunk) chunk_cnt[(int64_t)blockIdx.x * E + e] = cnt[e];
+}
+
+__global__ void __launch_bounds__(kChunk)
+    moe_route_count_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K,
+                           int E, MoeWs ws, int* __restrict__ chunk_cnt) {
+  route_count(ids, wts, B, K, E, ws, chunk_cnt);
+}
+__global__ void __launch_bounds__(kChunk)
+    moe_route_count_gated_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K,
+                                 int E, MoeWs ws, int* __restrict__ chunk_cnt, int nchunks, SharedGate gate) {
+  if (!gate_block(gate, nchunks)) route_count(ids, wts, B, K, E, ws, chunk_cnt);
 }
 
 // Scans over experts (lane e = expert e, whole waves of the workgroup; lanes
@@ -449,11 +460,9 @@ __global__ void __launch_bounds__(kMaxExperts)
 // placement with G lanes per token (so few tokens still spread over every
 // wave), the chunk's counts and positions kept in LDS (its offsets within
 // each expert are 0). Same outputs as the three launches.
-__global__ void __launch_bounds__(kMaxExperts)
-    moe_route_small_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K, int E,
-                           int mtile, MoeWs ws, SharedGate gate) {
+__device__ __forceinline__ void route_small(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B,
+                                            int K, int E, int mtile, const MoeWs& ws) {
   extern __shared__ int sm[];
-  if (gate_block(gate, 1)) return;
   int* s_ids = sm;                                                     // [kChunk * K]
   float* s_w = reinterpret_cast<float*>(sm + kChunk * K);              // [kChunk * K] staged weights
   float* s_m = reinterpret_cast<float*>(sm + 2 * kChunk * K);          // [kChunk * K] merged weights
@@ -504,6 +513,17 @@ __global__ void __launch_bounds__(kMaxExperts)
     else
       place_grp<32>(s_ids, s_m, bits, s_pos, b, g, G, K, b, tp, ws);
   }
+}
+
+__global__ void __launch_bounds__(kMaxExperts)
+    moe_route_small_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K, int E,
+                           int mtile, MoeWs ws) {
+  route_small(ids, wts, B, K, E, mtile, ws);
+}
+__global__ void __launch_bounds__(kMaxExperts)
+    moe_route_small_gated_kernel(const int32_t* __restrict__ ids, const uint16_t* __restrict__ wts, int B, int K, int E,
+                                 int mtile, MoeWs ws, SharedGate gate) {
+  if (!gate_block(gate, 1)) route_small(ids, wts, B, K, E, mtile, ws);
 }
 
 // ---------------------------------------------------------------------------
@@ -1642,12 +1662,13 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     // the count, 132 KB of staged rows, bitmaps and positions for the scatter
     const auto scatter_lds = [](int64_t k, int64_t e) { return (size_t)(3 * kChunk * k + e * (kChunkWords + 1)) * 4; };
     once_per_device(attr_done, [&] {
-      (void)hipFuncSetAttribute((const void*)moe_route_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kChunk * 32 * 8);
+      for (const void* k : {(const void*)moe_route_count_kernel, (const void*)moe_route_count_gated_kernel})
+        (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kChunk * 32 * 8);
       (void)hipFuncSetAttribute((const void*)moe_route_scatter_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)scatter_lds(32, kMaxExperts));
-      (void)hipFuncSetAttribute((const void*)moe_route_small_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)(scatter_lds(32, kMaxExperts) + kMaxExperts * 4));
+      for (const void* k : {(const void*)moe_route_small_kernel, (const void*)moe_route_small_gated_kernel})
+        (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(scatter_lds(32, kMaxExperts) + kMaxExperts * 4));
       (void)hipFuncSetAttribute((const void*)moe_route_scan_scatter_kernel,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)scatter_lds(32, kMaxExperts));
     });
@@ -1656,13 +1677,22 @@ static int moe_forward_impl(const q6moe_moe_args* a, void* workspace, size_t wor
     if (nchunks == 1) {
       // one chunk: the three passes in one launch (its counts and positions in LDS)
       const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);
-      const dim3 grid(1 + (unsigned)cdiv(gate.tokens, lanes / 64));
-      hipLaunchKernelGGL(moe_route_small_kernel, grid, dim3(lanes), scatter_lds(K, E) + (size_t)E * 4, s, a->ids,
-                         a->weights, (int)B, (int)K, (int)E, mtile, ws, gate);
+      const size_t lds = scatter_lds(K, E) + (size_t)E * 4;
+      if (gate.tokens)
+        hipLaunchKernelGGL(moe_route_small_gated_kernel, dim3(1 + (unsigned)cdiv(gate.tokens, lanes / 64)), dim3(lanes),
+                           lds, s, a->ids, a->weights, (int)B, (int)K, (int)E, mtile, ws, gate);
+      else
+        hipLaunchKernelGGL(moe_route_small_kernel, dim3(1), dim3(lanes), lds, s, a->ids, a->weights, (int)B, (int)K,
+                           (int)E, mtile, ws);
     } else {
-      const dim3 grid((unsigned)(nchunks + cdiv(gate.tokens, kChunk / 64)));
-      hipLaunchKernelGGL(moe_route_count_kernel, grid, dim3(kChunk), (size_t)kChunk * K * 8, s, a->ids, a->weights,
-                         (int)B, (int)K, (int)E, nchunks, ws, chunk_cnt, gate);
+      const size_t lds = (size_t)kChunk * K * 8;
+      if (gate.tokens)
+        hipLaunchKernelGGL(moe_route_count_gated_kernel, dim3((unsigned)(nchunks + cdiv(gate.tokens, kChunk / 64))),
+                           dim3(kChunk), lds, s, a->ids, a->weights, (int)B, (int)K, (int)E, ws, chunk_cnt, nchunks,
+                           gate);
+      else
+        hipLaunchKernelGGL(moe_route_count_kernel, dim3(nchunks), dim3(kChunk), lds, s, a->ids, a->weights, (int)B,
+                           (int)K, (int)E, ws, chunk_cnt);
       if (nchunks <= kFoldChunks) {
         // the scan folded into the scatter workgroups (up to 8192 tokens)
         const unsigned lanes = (unsigned)std::max<int64_t>(kChunk, cdiv(E, 64) * 64);

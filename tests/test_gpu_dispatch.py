@@ -52,23 +52,26 @@ def test_tile_width_by_format_and_routes_per_expert(device, kernels, qtype, down
             assert (", 64>" in name, ", 128>" in name) == (thin, not thin), (per, name)
 
 
-def test_decode_gate_up_without_a_gate_runs_without_its_items(device, kernels):
+@pytest.mark.parametrize("tokens,mode,gated", [
+    (3, 1, "moe_dec_gate_up_gated_kernel"), (3, 2, "moe_route_small_gated_kernel"),
+    (257, 2, "moe_route_count_gated_kernel")])
+def test_launches_without_a_gate_run_without_its_items(device, kernels, tokens, mode, gated):
     from q6moe.experts import expert_parallel, pack_experts
     from q6moe.synth import moe_layer
 
-    L = moe_layer(seed=4, experts=4, top_k=2, hidden=256, intermediate=256, tokens=3, shared_intermediate=256,
+    L = moe_layer(seed=4, experts=4, top_k=2, hidden=256, intermediate=256, tokens=tokens, shared_intermediate=256,
                   pack=False)
     fn = expert_parallel(None, gate_type="Q6_K", up_type="Q6_K", down_type="Q6_K", hidden=256, intermediate=256)
+    fn = fn.with_mode(mode)
     tabs = fn.prepare(*(L[n].reshape(4, -1) for n in ("gate", "up", "down")), device)
     sh = {n: pack_experts(L["shared"][n].reshape(1, -1), "Q6_K", 256, 256, device) for n in ("gate", "up", "down")}
     sh["intermediate"] = 256
     x = torch.from_numpy(L["x"]).to(device).to(torch.bfloat16)
     ids, w = torch.from_numpy(L["ids"]).to(device), torch.from_numpy(L["weights"]).to(device).to(torch.bfloat16)
     router = torch.ones(256, device=device, dtype=torch.bfloat16)
-    scale = torch.ones(3, device=device, dtype=torch.bfloat16)
-    for shared, gated in ((None, False), (sh, False), (dict(sh, scale=scale), False), (dict(sh, router=router), True)):
-        call = lambda: fn.with_mode(1)(*tabs, x, ids, w, shared=shared)  # noqa: E731
-        assert any("moe_dec_gate_up_gated_kernel" in k for k in kernels(call)) == gated
+    scale = torch.ones(tokens, device=device, dtype=torch.bfloat16)
+    for shared, gate in ((None, False), (sh, False), (dict(sh, scale=scale), False), (dict(sh, router=router), True)):
+        assert any(gated in k for k in kernels(lambda: fn(*tabs, x, ids, w, shared=shared))) == gate  # noqa: B023
 
 
 @pytest.mark.parametrize("qtype,down,experts,top_k,hidden,inter,shared,tokens,grouped", [
